@@ -90,6 +90,17 @@ int resident_grid(const void* kernel, int block, int fallback) {
   return ncu * per_cu;
 }
 
+// Compute units of the current device (256 if the runtime cannot say).
+int compute_units() {
+  int dev = 0, ncu = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) {
+    (void)hipGetLastError();
+    return 256;
+  }
+  return ncu;
+}
+
 #define TINA_HIP(ctx, call)                                   \
   do {                                                        \
     int _rc = hip_check((ctx), (call), #call);                \
@@ -363,12 +374,7 @@ int tina_ctx_create(int width, int height, int max_faces, tina_ctx** out) {
     release();
     return fail(nullptr, TINA_ERR_HIP, "counter initialisation failed");
   }
-  {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      c->ncu = 256;
-    (void)hipGetLastError();
-  }
+  c->ncu = compute_units();
   int rc = alloc_scratch(c, max_faces);
   if (rc != TINA_OK) {
     g_create_err = c->err;
@@ -761,8 +767,9 @@ int tina_bake_ibl(const float* d_env, int ew, int eh, float* d_out, int ow, int 
   const double r = (double)roughness;
   const double alpha2 = roughness < 0.0f ? -1.0 : fmax(0.0, r * r);
   const long n = (long)ow * oh;
-  hipLaunchKernelGGL(k_bake_ibl, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, d_env, ew, eh,
-                     d_out, ow, oh, alpha2, nsamples);
+  const int tpb = bake_tpb(n, compute_units());
+  hipLaunchKernelGGL(k_bake_ibl, dim3((unsigned)((n + tpb - 1) / tpb)), dim3(kBakeBlock), 0, (hipStream_t)stream,
+                     d_env, ew, eh, d_out, ow, oh, alpha2, nsamples, tpb);
   return hip_check(nullptr, hipGetLastError(), "k_bake_ibl");
 }
 
