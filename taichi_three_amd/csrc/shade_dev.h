@@ -19,8 +19,9 @@ __device__ __forceinline__ V3 vsub(V3 a, V3 b) { return v3(a.x - b.x, a.y - b.y,
 __device__ __forceinline__ V3 vmul(V3 a, V3 b) { return v3(a.x * b.x, a.y * b.y, a.z * b.z); }
 __device__ __forceinline__ V3 vsmul(float s, V3 a) { return v3(s * a.x, s * a.y, s * a.z); }
 __device__ __forceinline__ V3 vdivs(V3 a, float s) {
-  const RcpRN R = rcp_rn(s);
-  return v3(div_rn(a.x, R), div_rn(a.y, R), div_rn(a.z, R));
+  V3 q;
+  div3_rn(a.x, a.y, a.z, rcp_rn(s), q.x, q.y, q.z);
+  return q;
 }
 __device__ __forceinline__ V3 vneg(V3 a) { return v3(-a.x, -a.y, -a.z); }
 // a / d as a times the hardware reciprocal of d (v_rcp_f32, within 1 ulp), for
@@ -46,8 +47,9 @@ __device__ __forceinline__ V3 mapply_pos(const float* __restrict__ M, V3 p, floa
   float r0, r1, r2, w;
   mapply1(M, p.x, p.y, p.z, r0, r1, r2, w);
   if (wout) *wout = w;
-  const RcpRN R = rcp_rn(w);
-  return v3(div_rn(r0, R), div_rn(r1, R), div_rn(r2, R));
+  V3 q;
+  div3_rn(r0, r1, r2, rcp_rn(w), q.x, q.y, q.z);
+  return q;
 }
 
 // bilerp (tina/common.py:140-149) over a [w][h][c] array; the indices are
@@ -352,8 +354,10 @@ __device__ __forceinline__ void fragment(const ShadeArgs& a, uint32_t f, int px,
   const float cx = (Cv.x * 0.5f + 0.5f) * resx, cy = (Cv.y * 0.5f + 0.5f) * resy;
   const float nn = (bx - ax) * (cy - ay) - (by - ay) * (cx - ax);
   const RcpRN Rn = rcp_rn(nn);
-  const float bcnx = div_rn(bx - cx, Rn), bcny = div_rn(by - cy, Rn);
-  const float canx = div_rn(cx - ax, Rn), cany = div_rn(cy - ay, Rn);
+  const float e[4] = {bx - cx, by - cy, cx - ax, cy - ay};
+  float eq[4];
+  div_rn_n<4>(e, Rn, eq);
+  const float bcnx = eq[0], bcny = eq[1], canx = eq[2], cany = eq[3];
   const float ws0 = fdiv_rn(1.0f, wA), ws1 = fdiv_rn(1.0f, wB), ws2 = fdiv_rn(1.0f, wC);
   const float p_x = (float)px + a.cam.bias[0], p_y = (float)py + a.cam.bias[1];
   const float w_bc = (p_x - bx) * bcny - (p_y - by) * bcnx;
@@ -362,7 +366,7 @@ __device__ __forceinline__ void fragment(const ShadeArgs& a, uint32_t f, int px,
   float wx = w_bc * ws0, wy = w_ca * ws1, wz = t * ws2;
   const float s = (wx + wy) + wz;
   const RcpRN Rs = rcp_rn(s);
-  wx = div_rn(wx, Rs); wy = div_rn(wy, Rs); wz = div_rn(wz, Rs);
+  div3_rn(wx, wy, wz, Rs, wx, wy, wz);
   fr.w0 = wx; fr.w1 = wy; fr.w2 = wz;
 
   fr.pos = vadd(vadd(vsmul(wx, A), vsmul(wy, B)), vsmul(wz, C));

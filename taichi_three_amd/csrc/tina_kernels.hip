@@ -321,10 +321,17 @@ k_selftest_div(int mode, uint64_t npairs, uint32_t seed, unsigned long long* __r
     const RcpRN R = rcp_rn(d);
     const float aa = fabsf(a);
     fast += (R.ok & (aa >= 0x1p-60f) & (aa <= 0x1p60f)) ? 1u : 0u;
-    const float got = div_rn(a, R);
-    const float want = a / d;
-    const bool same = (__float_as_uint(got) == __float_as_uint(want)) || (got != got && want != want);
-    bad += same ? 0u : 1u;
+    auto same = [](float got, float want) {
+      return (__float_as_uint(got) == __float_as_uint(want)) || (got != got && want != want);
+    };
+    // the grouped form, beside a numerator of another pair and an ordinary one
+    const float other = mode == 1 ? __builtin_canonicalizef(__uint_as_float(h(ab ^ 0x27d4eb2du))) : 1.5f;
+    float g0, g1, g2;
+    div3_rn(__builtin_canonicalizef(a), other, 0.75f, R, g0, g1, g2);
+    bad += same(div_rn(a, R), a / d) && same(g0, a / d) && same(g1, other / d) &&
+                   same(g2, 0.75f / d)
+               ? 0u
+               : 1u;
   }
   atomicAdd(&counts[0], fast);
   atomicAdd(&counts[1], bad);
