@@ -51,6 +51,7 @@ struct tina_ctx {
   uint32_t* fbn = nullptr;
   long fb_segcap = 0;
   int nn_grid = 0;
+  uint32_t* span = nullptr;       // the coarse depth table k_ssr reads, rebuilt by every tina_ssr
   // tina_clear only records the clear; the next call that touches the keys applies it
   // (the binned raster by starting its tiles from empty keys, anything else with
   // k_clear first)
@@ -360,7 +361,7 @@ int tina_ctx_create(int width, int height, int max_faces, tina_ctx** out) {
   c->cam.W2V[10] = c->cam.V2W[10] = -1.0f;
   c->cam.bias[0] = c->cam.bias[1] = 0.5f;
   auto release = [c]() {
-    for (void* p : {(void*)c->keys, (void*)c->ctr, (void*)c->cursor, (void*)c->fbq, (void*)c->fbn})
+    for (void* p : {(void*)c->keys, (void*)c->ctr, (void*)c->cursor, (void*)c->fbq, (void*)c->fbn, (void*)c->span})
       if (p) (void)hipFree(p);
     delete c;
   };
@@ -370,7 +371,8 @@ int tina_ctx_create(int width, int height, int max_faces, tina_ctx** out) {
   if (hipMalloc(&c->keys, sizeof(uint64_t) * (size_t)width * height) != hipSuccess ||
       hipMalloc(&c->ctr, sizeof(Counters)) != hipSuccess || hipMalloc(&c->cursor, sizeof(uint32_t)) != hipSuccess ||
       hipMalloc(&c->fbq, sizeof(uint32_t) * (size_t)c->fb_segcap * kFbSeg) != hipSuccess ||
-      hipMalloc(&c->fbn, sizeof(uint32_t) * kFbWords) != hipSuccess) {
+      hipMalloc(&c->fbn, sizeof(uint32_t) * kFbWords) != hipSuccess ||
+      hipMalloc(&c->span, sizeof(uint32_t) * (size_t)span_words(width, height)) != hipSuccess) {
     (void)hipGetLastError();
     release();
     return fail(nullptr, TINA_ERR_ALLOC, "hipMalloc of the depth|id buffer failed");
@@ -396,7 +398,7 @@ int tina_ctx_create(int width, int height, int max_faces, tina_ctx** out) {
 int tina_ctx_destroy(tina_ctx* c) {
   if (!c) return TINA_OK;
   free_scratch(c);
-  for (void* p : {(void*)c->keys, (void*)c->ctr, (void*)c->cursor, (void*)c->fbq, (void*)c->fbn})
+  for (void* p : {(void*)c->keys, (void*)c->ctr, (void*)c->cursor, (void*)c->fbq, (void*)c->fbn, (void*)c->span})
     if (p) (void)hipFree(p);
   delete c;
   return TINA_OK;
@@ -643,10 +645,10 @@ int tina_ssr(tina_ctx* c, const tina_mesh* mesh, const tina_material* mat, const
   sa.taa = taa ? 1 : 0;
   sa.stepsize = stepsize;
   sa.tolerance = tolerance;
+  sa.span = c->span;
+  sa.span_log = span_log(c->W, c->H);
   sa.seed = seed;
-  const long npix = (long)c->W * c->H;
-  hipLaunchKernelGGL(k_ssr, dim3(grid_for(npix, kBlock, 8192)), dim3(kBlock), 0, (hipStream_t)stream, a,
-                     (const uint64_t*)c->keys, sa);
+  dispatch_ssr(classify_program(a.mat, false), c->W, c->H, (hipStream_t)stream, a, c->keys, sa);
   TINA_LAUNCH(c, "k_ssr");
   return TINA_OK;
 }
