@@ -1013,8 +1013,8 @@ int tina_dshade_backward(tina_ctx* c, const tina_dmesh* m, const tina_lights* li
   int rc = make_diff_args(c, m, lights, A);
   if (rc) return rc;
   if ((rc = flush_clear(c, (hipStream_t)stream))) return rc;
-  const long npix = (long)c->W * c->H;
-  hipLaunchKernelGGL(k_dshade_bwd, dim3(grid_for(npix, kBlock, 0x7fffffff)), dim3(kBlock), 0, (hipStream_t)stream,
+  const long ntiles = (long)((c->W + kDiffTile - 1) / kDiffTile) * ((c->H + kDiffTile - 1) / kDiffTile);
+  hipLaunchKernelGGL(k_dshade_bwd, dim3((unsigned)std::min(ntiles, kDiffGridPerCu * (long)c->ncu)), dim3(kBlock), 0, (hipStream_t)stream,
                      A, c->keys, d_gimg, (float*)g->colors, (float*)g->normals, (float*)g->rough, (float*)g->metal,
                      (float*)g->intensity);
   TINA_LAUNCH(c, "k_dshade_bwd");
