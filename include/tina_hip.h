@@ -198,6 +198,12 @@ int tina_raster_particles(tina_ctx *ctx, const float *d_pos, const float *d_radi
  * wire whose two end points both leave the view cube (wireframe.py:75-78). */
 int tina_raster_wires(tina_ctx *ctx, const float *d_verts, int n, uint32_t id_base, uint32_t flags,
                       void *stream);
+/* Makes the scratch with which tina_raster_wires takes calls of n wires by screen
+ * tiles (65,536 wires and more; fewer need none, and without it, or where the memory
+ * is short, they are drawn into the depth|id buffer directly, with the same result).
+ * Made once per context, at most 60 MB at 1920 x 1080; nothing is made while stream
+ * is capturing.  Call it where the wires are bound, outside the frame. */
+int tina_wires_reserve(tina_ctx *ctx, int n, void *stream);
 
 /* The colour pass of WireframeRaster (wireframe.py:92-95, Shader.blend_color
  * with factor 1): every pixel whose winning id lies in [id_base, id_base + n)

@@ -124,6 +124,7 @@ EXPORTS = [
     ('tina_raster', _i32, [_vp, _vp, _i32, _u32, _u32, _vp]),
     ('tina_raster_particles', _i32, [_vp, _vp, _vp, _i32, _u32, _u32, _vp]),
     ('tina_raster_wires', _i32, [_vp, _vp, _i32, _u32, _u32, _vp]),
+    ('tina_wires_reserve', _i32, [_vp, _i32, _vp]),
     ('tina_paint_ids', _i32, [_vp, _u32, _i32, _vp, _vp, _u32, _vp, _vp]),
     ('tina_normals', _i32, [_vp, ctypes.POINTER(Mesh), _u32, _vp, _vp]),
     ('tina_gbuffer', _i32, [_vp, ctypes.POINTER(Mesh), _u32, _i32, _i32, _vp, ctypes.c_float, _vp, _vp]),

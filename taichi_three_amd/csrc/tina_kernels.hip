@@ -45,6 +45,7 @@ struct tina_ctx {
   uint32_t* cursor = nullptr;     // the binning groups' entry cursor (zero between calls)
   FaceRec* recs = nullptr;
   int ncu = 0;                    // compute units of the device
+  void* wires = nullptr;          // scratch of wire calls by tile (WireScratch), or none
   // learned-shading fallback queue (kFbSeg segments of fb_segcap pixel indices),
   // its segment counters, and k_shade_nn's resident grid
   uint32_t* fbq = nullptr;
@@ -136,6 +137,7 @@ unsigned grid_for(long n, long per_block, unsigned cap) {
 void allow_big_lds() {
   static const bool done = [] {
     (void)hipFuncSetAttribute((const void*)k_bin, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBudget);
+    (void)hipFuncSetAttribute((const void*)k_wire_bin, hipFuncAttributeMaxDynamicSharedMemorySize, kWireLds);
     (void)hipFuncSetAttribute((const void*)k_bbin, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBudget);
     (void)hipGetLastError();
     return true;
@@ -361,7 +363,7 @@ int tina_ctx_create(int width, int height, int max_faces, tina_ctx** out) {
   c->cam.W2V[10] = c->cam.V2W[10] = -1.0f;
   c->cam.bias[0] = c->cam.bias[1] = 0.5f;
   auto release = [c]() {
-    for (void* p : {(void*)c->keys, (void*)c->ctr, (void*)c->cursor, (void*)c->fbq, (void*)c->fbn, (void*)c->span})
+    for (void* p : {(void*)c->keys, (void*)c->ctr, (void*)c->cursor, (void*)c->fbq, (void*)c->fbn, (void*)c->span, c->wires})
       if (p) (void)hipFree(p);
     delete c;
   };
@@ -398,7 +400,7 @@ int tina_ctx_create(int width, int height, int max_faces, tina_ctx** out) {
 int tina_ctx_destroy(tina_ctx* c) {
   if (!c) return TINA_OK;
   free_scratch(c);
-  for (void* p : {(void*)c->keys, (void*)c->ctr, (void*)c->cursor, (void*)c->fbq, (void*)c->fbn, (void*)c->span})
+  for (void* p : {(void*)c->keys, (void*)c->ctr, (void*)c->cursor, (void*)c->fbq, (void*)c->fbn, (void*)c->span, c->wires})
     if (p) (void)hipFree(p);
   delete c;
   return TINA_OK;
@@ -517,10 +519,55 @@ int tina_raster_wires(tina_ctx* c, const float* d_verts, int n, uint32_t id_base
   hipStream_t s = (hipStream_t)stream;
   int rc = flush_clear(c, s);
   if (rc) return rc;
-  constexpr int per_block = kBlock / kWireWalkWaves;
-  hipLaunchKernelGGL(k_wires, dim3(grid_for(n, per_block, 16384)), dim3(kBlock), 0, s, d_verts, n, id_base, flags,
-                     make_cam(c), (unsigned long long*)c->keys);
+  if (c->wires && wires_by_tile(n)) {
+    const WireScratch w = wire_scratch(c->W, c->H, c->ncu);
+    WireJob j;
+    wire_scratch_at(w, c->wires, j);
+    j.keys = c->keys;
+    j.cam = make_cam(c);
+    j.flags = flags;
+    allow_big_lds();
+    for (int f0 = 0; f0 < n; f0 += w.room) {
+      j.verts = d_verts + 6 * (size_t)f0;
+      j.n = std::min(n - f0, w.room);
+      j.id_base = id_base + (uint32_t)f0;
+      j.per = std::max((j.n + c->ncu - 1) / c->ncu, 64);
+      j.ngroups = (j.n + j.per - 1) / j.per;
+      hipLaunchKernelGGL(k_wire_bin, dim3(j.ngroups), dim3(kBinBlock), (size_t)j.ntiles * 4, s, j);
+      TINA_LAUNCH(c, "k_wire_bin");
+      launch_wire_tile(j, c->ncu, s);
+      TINA_LAUNCH(c, "k_wire_tile");
+    }
+    return TINA_OK;
+  }
+  const int per = wires_per_wave(n, c->ncu);
+  hipLaunchKernelGGL(k_wires, dim3(grid_for(n, (long)per * (kBlock / 64), 16384)), dim3(kBlock), 0, s, d_verts, n, per,
+                     id_base, flags, make_cam(c), (unsigned long long*)c->keys);
   TINA_LAUNCH(c, "k_wires");
+  return TINA_OK;
+}
+
+int tina_wires_reserve(tina_ctx* c, int n, void* stream) {
+  if (!c) return fail(nullptr, TINA_ERR_INVALID, "ctx is NULL");
+  if (n < 0) return fail(c, TINA_ERR_INVALID, "n must be >= 0");
+  if (c->wires || !wires_by_tile(n)) return TINA_OK;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return TINA_OK;  // no allocation while a graph is recorded: the wires are drawn
+  }
+  const WireScratch w = wire_scratch(c->W, c->H, c->ncu);
+  if (w.bytes == 0) return TINA_OK;
+  void* p = nullptr;
+  if (hipMalloc(&p, w.bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return TINA_OK;  // the wires are drawn
+  }
+  if (hipMemset(p, 0, kWireWords * sizeof(uint32_t)) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+    (void)hipFree(p);
+    return fail(c, TINA_ERR_HIP, "the wire scratch could not be cleared");
+  }
+  c->wires = p;
   return TINA_OK;
 }
 

@@ -3,15 +3,18 @@
 //   k_wires   the samples draw_line steps along each wire's screen segment
 //             (one pixel per step on the major axis, :50-64) enter the depth|id
 //             min with the depth interpolated by the 1/w weights of :83-91.
-//             Wires go in groups of 64 like particles: a lane sets one up, the
-//             wave scans the sample counts, and four waves walk the samples.
-//             Only the samples whose major-axis position can land on the screen
-//             are walked (the range is found in binary64 with a margin far above
-//             the binary32 rounding of a + k i + bias); each walked sample is
-//             evaluated and tested exactly as the reference evaluates it.
+//             A lane sets a wire up, the wave scans the sample counts and walks
+//             the samples, one a lane.  Only the samples whose major-axis position
+//             can land on the screen are walked (the range is found in binary64
+//             with a margin far above the binary32 rounding of a + k i + bias);
+//             each walked sample is evaluated and tested exactly as the reference
+//             evaluates it.
+//   k_wire_bin, k_wire_tile   the same samples, tile by tile of the screen with
+//             the keys in LDS, for calls of many wires.
 //   k_paint   blend_color with factor 1 (tina/core/shader.py:134-135): the pixels
 //             a range of ids won take one colour (the wire colour).
 #pragma once
+#include "bin_kernels.h"
 #include "shade_dev.h"
 
 namespace tina {
@@ -107,73 +110,525 @@ __device__ __forceinline__ bool wire_step(const Cam& cam, const WSetup& s, long 
   return true;
 }
 
-constexpr int kWireWalkWaves = 4;
-
-__global__ void __launch_bounds__(kBlock)
-k_wires(const float* __restrict__ verts, int n, uint32_t id_base, uint32_t flags, const Cam cam,
-        unsigned long long* __restrict__ keys) {
-  constexpr int GW = kWireWalkWaves, NG = (kBlock / 64) / GW;
-  __shared__ uint64_t s_pre[64 * NG];
-  __shared__ uint64_t s_tot[NG];
-  __shared__ float s_f[8][64 * NG];  // ax ay kx ky ws0 ws1 Az Bz
-  __shared__ int32_t s_siz[64 * NG], s_i0[64 * NG];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const bool clip = (flags & TINA_CLIP) != 0;
-  gf32* gv = (gf32*)verts;
-  for (long bb = (long)blockIdx.x * 64 * NG; bb < n; bb += (long)gridDim.x * 64 * NG) {
-    WSetup s;
-    uint64_t cnt = 0;
-    if (t < 64 * NG && bb + t < n && !wire_setup(cam, gv, bb + t, clip, s, cnt)) cnt = 0;
-    uint64_t inc = cnt;
+// Draws the wires of a wave's lanes (count steps of s each) into memory, the steps
+// laid end to end, one a lane.  The first slot whose end is beyond step g owns it:
+// the slots that ended before the window of 64, and the ends marked in it below the
+// lane.  mark, slot: LDS of the wave's own, 64 words each, mark at -1.
+__device__ __forceinline__ void wires_to_memory(const Cam& cam, const WSetup& s, uint64_t count, uint32_t id,
+                                                unsigned long long* __restrict__ keys, int* mark, int* slot) {
+  const int lane = __lane_id();
+  const unsigned long long live = __ballot(count > 0);
+  uint64_t end = count;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const uint64_t u = __shfl_up(inc, d, 64);
-      if (lane >= d) inc += u;
-    }
-    __syncthreads();  // the previous pass's readers are done with the tables
-    if (t < 64 * NG) {
-      s_pre[t] = inc - cnt;
-      if (lane == 63) s_tot[wave] = inc;
-      if (cnt) {
-        s_f[0][t] = s.ax;
-        s_f[1][t] = s.ay;
-        s_f[2][t] = s.kx;
-        s_f[3][t] = s.ky;
-        s_f[4][t] = s.ws0;
-        s_f[5][t] = s.ws1;
-        s_f[6][t] = s.Az;
-        s_f[7][t] = s.Bz;
-        s_siz[t] = s.siz;
-        s_i0[t] = s.i0;
-      }
-    }
-    __syncthreads();
-    const int gb = (wave / GW) * 64;
-    const uint64_t total = s_tot[wave / GW];
-    for (uint64_t k = (uint64_t)((wave % GW) * 64 + lane); k < total; k += 64 * GW) {
-      int lo = 0;
-#pragma unroll
-      for (int step = 32; step > 0; step >>= 1)
-        if (s_pre[gb + lo + step] <= k) lo += step;
-      const int j = gb + lo;
-      WSetup q;
-      q.ax = s_f[0][j];
-      q.ay = s_f[1][j];
-      q.kx = s_f[2][j];
-      q.ky = s_f[3][j];
-      q.ws0 = s_f[4][j];
-      q.ws1 = s_f[5][j];
-      q.Az = s_f[6][j];
-      q.Bz = s_f[7][j];
-      q.siz = s_siz[j];
-      int X, Y;
-      int32_t depth;
-      if (!wire_step(cam, q, (long)s_i0[j] + (long)(k - s_pre[j]), X, Y, depth)) continue;
-      const unsigned long long key = pack_key(depth, id_base + (uint32_t)(bb + j));
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint64_t u = __shfl_up(end, d, 64);
+    if (lane >= d) end += u;
+  }
+  const uint64_t total = __shfl(end, 63, 64);
+  auto below = [&](unsigned long long m) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+  };
+  if (count > 0) slot[below(live)] = lane;
+  int kbase = 0, tag = 0;
+  for (uint64_t g0 = 0; g0 < total; g0 += 64) {
+    // windows are told apart by 31 bits of their number: a mark is read in its own
+    tag = (tag + 1) & 0x7fffffff;
+    if (count > 0 && end - 1 >= g0 && end - 1 < g0 + 64) mark[(int)(end - 1 - g0)] = tag;
+    wave_sync_lds();
+    const unsigned long long ends = __ballot(mark[lane] == tag);
+    const uint64_t g = g0 + lane;
+    const int j = g < total ? slot[kbase + below(ends)] : lane;
+    kbase += __popcll(ends);
+    WSetup q;
+    q.ax = __shfl(s.ax, j);
+    q.ay = __shfl(s.ay, j);
+    q.kx = __shfl(s.kx, j);
+    q.ky = __shfl(s.ky, j);
+    q.ws0 = __shfl(s.ws0, j);
+    q.ws1 = __shfl(s.ws1, j);
+    q.Az = __shfl(s.Az, j);
+    q.Bz = __shfl(s.Bz, j);
+    q.siz = __shfl(s.siz, j);
+    const int64_t i = (int64_t)g + __shfl((int64_t)s.i0 - (int64_t)(end - count), j);
+    const uint32_t idj = __shfl(id, j);
+    int X, Y;
+    int32_t depth;
+    if (g < total && wire_step(cam, q, (long)i, X, Y, depth)) {
+      const unsigned long long key = pack_key(depth, idj);
       unsigned long long* kp = keys + (long)Y * cam.W + X;
       if (key < __hip_atomic_load(kp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(kp, key);
     }
+    wave_sync_lds();
   }
+  if (count > 0 || mark[lane] != -1) mark[lane] = -1;
+  wave_sync_lds();
+}
+
+// Every wire into memory, `per` (at most 64) wires a wave at a time.
+__global__ void __launch_bounds__(kBlock)
+k_wires(const float* __restrict__ verts, int n, int per, uint32_t id_base, uint32_t flags, const Cam cam,
+        unsigned long long* __restrict__ keys) {
+  __shared__ int s_mark[kBlock], s_slot[kBlock];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool clip = (flags & TINA_CLIP) != 0;
+  s_mark[threadIdx.x] = -1;
+  for (long f0 = ((long)blockIdx.x * (kBlock / 64) + wave) * per; f0 < n; f0 += (long)gridDim.x * (kBlock / 64) * per) {
+    WSetup s;
+    s.ax = s.ay = s.kx = s.ky = s.ws0 = s.ws1 = s.Az = s.Bz = 0.0f;
+    s.siz = s.i0 = 0;
+    uint64_t cnt = 0;
+    const long f = f0 + lane;
+    if (lane < per && f < n && !wire_setup(cam, (gf32*)verts, f, clip, s, cnt)) cnt = 0;
+    wires_to_memory(cam, s, cnt, id_base + (uint32_t)f, keys, s_mark + 64 * wave, s_slot + 64 * wave);
+  }
+}
+
+// Wires a wave for a call of n: 64 waves a CU (eight of them at a time) before a
+// wave takes a second wire.  Against 16 waves a CU: 32 k long wires 256 us for 268,
+// 200 k of 2 px 50 for 47; 64 wires a wave, as before, left 500 wires of 600 px with
+// eight workgroups (147 us; 39 now).
+inline int wires_per_wave(long n, int ncu) {
+  const long p = (n + 64L * ncu - 1) / (64L * ncu);
+  return (int)(p < 1 ? 1 : p > 64 ? 64 : p);
+}
+
+// ---- wires by tile ---------------------------------------------------------------
+//
+// Each wire's steps land on keys all over the screen, so drawing into memory is
+// bound by L2 (a line a step; the 16.6 MB of keys of a 1080p screen do not fit an
+// XCD's 4 MB) and by 64-bit atomics (27 G/s).  Calls of many wires therefore go by
+// tiles of 32 x 32 pixels whose keys sit in LDS: k_wire_bin lists the wires of
+// every tile, k_wire_tile walks each tile's.  What bounds it then is VALU issue in
+// the tile pass (about 45 instructions a step, 70 % of its time) and the tiles over
+// the middle of the screen, which hold most entries.
+// 200 k random wires of 600 px at 1080p: 800 us in memory, 317 by tile (k_wire_bin
+// 60, k_wire_tile 257; tiles of 16 pixels 355, of 64 400).  Two workgroups a CU take
+// tiles in turn: a workgroup per tile is as fast, but 4.8 us for 2.5 when all groups
+// have drawn their wires.
+constexpr int kWireTileLog = 5, kWireTile = 1 << kWireTileLog;
+
+// Calls of this many wires go by tile where their steps are many (kWireGroupSteps).
+// Frames of 1080p with 66 k wires of 600, 150, 50, 15 and 5 px: 408 -> 177 us, 151 ->
+// 104, 80 -> 81, 45 -> 49, 38 -> 40; with 200 k: 818 -> 325, 279 -> 128, 146 -> 98, 76
+// -> 81, 49 -> 54 (at 800 x 450, a third as long: 360 -> 265, 142 -> 72, 82 -> 89, 43 ->
+// 53).  The steps are counted on the device, so a call of short wires pays the tile
+// pass's empty launch and a raster by k_wire_bin, at half of k_wires's waves.  Below
+// this count short wires are the usual ones and the launch is the same price (16 k of
+// 50 px 39 -> 44).
+constexpr int kWireTiledCall = 65536;
+inline bool wires_by_tile(long n) { return n >= kWireTiledCall; }
+
+// A wire's set-up, one cache line.
+struct WireRec {
+  float4 a;  // ax, ay, kx, ky
+  float4 b;  // ws0, ws1, Az, Bz
+  float4 c;  // integers: siz, first and last walked step (none: last < first), then e (below)
+  float4 d;  // n0, n1, d0, d1: step i's z is about (n0 + n1 i) / (d0 + d1 i)
+};
+
+struct WireJob {
+  const float* verts;
+  uint64_t* keys;
+  uint32_t* chunk_off;
+  uint32_t* chunk_cnt;
+  uint32_t* entries;
+  WireRec* recs;
+  uint32_t* gcnt;     // [ngroups] entries of each group
+  uint32_t* cursor;   // entries reserved, then the tile pass's next tile (kWireWords)
+  Cam cam;
+  int n;
+  uint32_t id_base, flags, cap;  // cap: entries there is room for
+  int tiles_x, ntiles, ngroups, per;  // per: wires a group
+};
+
+// Scratch of wire calls by tile: one allocation, kept by the context once a call's
+// count asks for it.  kWireRoom wires go at a time and have kWireEntries entries each
+// (wires of 600 px have about 22); a table of counts and one of offsets for as many
+// groups as the device has units.  1080p: 46 MB.
+constexpr int kWireLds = kLdsBudget - 16 * 1024;  // for k_wire_bin's counts by tile (its static LDS is 9 KB)
+constexpr int kWireRoom = 262144, kWireEntries = 24, kWireWords = 2;
+struct WireScratch {
+  int tiles_x, ntiles, room;
+  size_t gcnt, chunk_cnt, chunk_off, entries, recs, bytes;  // places in bytes; the cursor's words come first
+};
+
+inline WireScratch wire_scratch(int W, int H, int ncu) {
+  WireScratch w;
+  w.tiles_x = (W + kWireTile - 1) / kWireTile;
+  const long ntiles = (long)w.tiles_x * ((H + kWireTile - 1) / kWireTile);
+  w.bytes = 0;
+  if (4 * ntiles > kWireLds) return w;
+  w.ntiles = (int)ntiles;
+  // the count of all entries, at most a few tile rows and columns a wire, has 32 bits
+  w.room = (int)std::min((long)kWireRoom, 0xFFFFFFFFL / (4L * (w.tiles_x + ntiles / w.tiles_x + 4)));
+  auto place = [&](size_t n) {
+    const size_t at = w.bytes;
+    w.bytes += (n + 255) & ~(size_t)255;
+    return at;
+  };
+  place(4 * (size_t)kWireWords);
+  w.gcnt = place(4 * (size_t)ncu);
+  w.chunk_cnt = place(4 * (size_t)ncu * w.ntiles);
+  w.chunk_off = place(4 * (size_t)ncu * w.ntiles);
+  w.entries = place(4 * (size_t)kWireRoom * kWireEntries);
+  w.recs = place(sizeof(WireRec) * (size_t)kWireRoom);
+  return w;
+}
+
+inline void wire_scratch_at(const WireScratch& w, void* base, WireJob& j) {
+  char* const b = (char*)base;
+  j.cursor = (uint32_t*)b;
+  j.gcnt = (uint32_t*)(b + w.gcnt);
+  j.chunk_cnt = (uint32_t*)(b + w.chunk_cnt);
+  j.chunk_off = (uint32_t*)(b + w.chunk_off);
+  j.entries = (uint32_t*)(b + w.entries);
+  j.recs = (WireRec*)(b + w.recs);
+  j.cap = (uint32_t)(kWireRoom * kWireEntries);
+  j.tiles_x = w.tiles_x;
+  j.ntiles = w.ntiles;
+}
+
+// Bound on the distance of the binary32 a + k i + bias of a walked step from its
+// exact value: three roundings of at most the magnitudes involved (2^-24 each).
+__device__ __forceinline__ double wire_axis_err(float a, float k, int siz, float bias) {
+  return 1e-3 + 1e-6 * (fabs((double)a) + fabs((double)k) * (double)siz + fabs((double)bias));
+}
+
+// Narrows the steps [lo, hi] to those whose exact position p0 + k i (p0 = a + bias)
+// lies within err of [q0, q1].
+__device__ __forceinline__ void wire_clip(double p0, double k, double q0, double q1, double err, double& lo, double& hi) {
+  const double l = q0 - err - p0, h = q1 + err - p0;
+  if (k == 0.0) {
+    if (l > 0.0 || h < 0.0) hi = lo - 1.0;
+    return;
+  }
+  const double ik = 1.0 / k, i0 = l * ik, i1 = h * ik;
+  lo = fmax(lo, fmin(i0, i1));
+  hi = fmin(hi, fmax(i0, i1));
+}
+
+// Every tile a walked step of the wire can fall in (and a few beside it): along the
+// major axis a tile at a time, the tiles its steps there can reach on the other.
+template <class F>
+__device__ __forceinline__ void wire_tiles(const WireJob& j, const WireRec& r, F&& visit) {
+  const bool xm = fabsf(r.a.z) == 1.0f;  // unit steps along x
+  const float bx = j.cam.bias[0], by = j.cam.bias[1];
+  const int siz = __float_as_int(r.c.x), tx = j.tiles_x, ty = j.ntiles / j.tiles_x;
+  const double ex = wire_axis_err(r.a.x, r.a.z, siz, bx), ey = wire_axis_err(r.a.y, r.a.w, siz, by);
+  const double px = (double)r.a.x + (double)bx, py = (double)r.a.y + (double)by;
+  const double pm = xm ? px : py, km = xm ? r.a.z : r.a.w, em = xm ? ex : ey;
+  const double pn = xm ? py : px, kn = xm ? r.a.w : r.a.z, en = xm ? ey : ex;
+  const double lo = __float_as_int(r.c.y), hi = __float_as_int(r.c.z), tile = kWireTile, inv = 1.0 / kWireTile;
+  const int nm = xm ? tx : ty, nn = xm ? ty : tx;
+  const double m0 = pm + km * lo, m1 = pm + km * hi;
+  const int c0 = (int)fmin(fmax(floor((fmin(m0, m1) - em) * inv), 0.0), (double)nm);
+  const int c1 = (int)fmin(fmax(floor((fmax(m0, m1) + em) * inv), -1.0), (double)(nm - 1));
+  for (int c = c0; c <= c1; c++) {
+    double l = lo, h = hi;
+    wire_clip(pm, km, tile * c, tile * (c + 1), em, l, h);
+    if (!(l <= h)) continue;
+    const double y0 = pn + kn * l, y1 = pn + kn * h;
+    const int r0 = (int)fmin(fmax(floor((fmin(y0, y1) - en) * inv), 0.0), (double)nn);
+    const int r1 = (int)fmin(fmax(floor((fmax(y0, y1) + en) * inv), -1.0), (double)(nn - 1));
+    for (int q = r0; q <= r1; q++) visit(xm ? q * tx + c : c * tx + q);
+  }
+}
+
+// Steps of a round of up to 1,024 wires from which they are listed by tile instead
+// of drawn: about 3 M a call, where the two meet (128 k wires of 50 px, 6.4 M steps:
+// 92 us by tile, 113 in memory; 64 k, 3.2 M: 82 either way; twice the limit leaves
+// 64 k of 150 px at 150 instead of 103).
+constexpr uint64_t kWireGroupSteps = 12288;
+
+// Group blockIdx.x's wires, up to 1,024 at a time (pw by each of the sixteen waves):
+// set up, then, where their steps are many, counted per tile and, once the group is
+// through, listed per tile (as bin_group does for faces); where they are few, drawn
+// into memory, so that the tile pass finds nothing to do.  Wires with no length or a
+// value that is not finite, which have no tiles to find, are drawn, as are all of a
+// group whose entries do not fit.
+__global__ void __launch_bounds__(kBinBlock) k_wire_bin(const WireJob jv) {
+  TINA_KERNARG_JOB(WireJob, j, jv);
+  extern __shared__ __align__(16) uint32_t lds[];
+  uint32_t* const cnt = lds;  // [ntiles] counts, then running offsets
+  __shared__ unsigned long long s_steps;
+  __shared__ uint32_t s_base, s_carry, s_wsum[kBinBlock / 64];
+  __shared__ int s_mark[kBinBlock], s_slot[kBinBlock];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wbase = tid & ~63, ntiles = j.ntiles;
+  constexpr int kWaves = kBinBlock / 64;
+  const int pw = min(64, (j.per + kWaves - 1) / kWaves);
+  const long f0 = (long)blockIdx.x * j.per, f1 = min((long)j.n, f0 + j.per), round = (long)kWaves * pw;
+  const bool clip = (j.flags & TINA_CLIP) != 0;
+  unsigned long long* const keys = (unsigned long long*)j.keys;
+  // this lane's wire of the round at b
+  auto mine = [&](long b) { return lane < pw ? b + wave * pw + lane : f1; };
+  auto draw = [&](const WSetup& s, uint64_t steps, long f) {
+    if (__any(steps > 0)) wires_to_memory(j.cam, s, steps, j.id_base + (uint32_t)f, keys, s_mark + wbase, s_slot + wbase);
+  };
+  s_mark[tid] = -1;
+  if (blockIdx.x == 0 && tid == 0) j.cursor[1] = 0u;  // the tile pass's next tile
+  bool listed = false;  // uniform: some round of the group goes by tile
+  for (long b = f0; b < f1; b += round) {
+    const long f = mine(b);
+    if (tid == 0) s_steps = 0;
+    __syncthreads();
+    WSetup s;
+    s.ax = s.ay = s.kx = s.ky = s.ws0 = s.ws1 = s.Az = s.Bz = 0.0f;
+    s.siz = s.i0 = 0;
+    uint64_t steps = 0;
+    if (f < f1 && !wire_setup(j.cam, (gf32*)j.verts, f, clip, s, steps)) steps = 0;
+    if (steps) atomicAdd(&s_steps, (unsigned long long)steps);
+    __syncthreads();
+    const bool tiled = s_steps >= kWireGroupSteps;
+    if (tiled && !listed) {
+      listed = true;
+      for (int t = tid; t < ntiles; t += kBinBlock) cnt[t] = 0;
+      __syncthreads();
+    }
+    const float sum = ((fabsf(s.ax) + fabsf(s.ay)) + (fabsf(s.kx) + fabsf(s.ky))) +
+                      ((fabsf(s.ws0) + fabsf(s.ws1)) + (fabsf(s.Az) + fabsf(s.Bz)));
+    const bool list = tiled && steps > 0 && s.siz > 0 && sum < 1e9f;
+    WireRec r;
+    if (list) {
+      r.a = make_float4(s.ax, s.ay, s.kx, s.ky);
+      r.b = make_float4(s.ws0, s.ws1, s.Az, s.Bz);
+      // z by steps: n / d with n = ws0 Az (1 - c) + ws1 Bz c, d = ws0 (1 - c) + ws1 c, c = i / siz
+      const float is = 1.0f / (float)s.siz, n0 = s.ws0 * s.Az, d0 = s.ws0;
+      r.d = make_float4(n0, (s.ws1 * s.Bz - n0) * is, d0, (s.ws1 - d0) * is);
+      // e: z d computed so, and the reference's own z, are off by less than e (32 roundings
+      // of the largest terms); both ends in front of the camera, or no bound
+      const float mx = fmaxf(s.ws0, s.ws1), mn = fminf(s.ws0, s.ws1);
+      const float e = 32.0f * 5.9604645e-8f * mx * (1.0f + fmaxf(fabsf(s.Az), fabsf(s.Bz))) * (1.0f + mx / mn);
+      r.c = make_float4(__int_as_float(s.siz), __int_as_float(s.i0),
+                        __int_as_float((int)((int64_t)s.i0 + (int64_t)steps - 1)), mn > 0.0f ? e : INFINITY);
+      wire_tiles(j, r, [&](int t) { atomicAdd(&cnt[t], 1u); });
+      j.recs[f] = r;
+    } else if (f < f1 && (tiled || j.per > round)) {
+      j.recs[f].c = make_float4(0.0f, __int_as_float(0), __int_as_float(-1), 0.0f);  // not listed
+    }
+    draw(s, list ? 0 : steps, f);
+  }
+  if (!listed) {  // the tile pass takes no counts from this group
+    if (tid == 0) j.gcnt[blockIdx.x] = 0u;
+    return;
+  }
+  __syncthreads();
+  uint32_t* __restrict__ chunk_cnt = j.chunk_cnt + (size_t)blockIdx.x * ntiles;
+  uint32_t* __restrict__ chunk_off = j.chunk_off + (size_t)blockIdx.x * ntiles;
+  for (int t = tid; t < ntiles; t += kBinBlock) chunk_cnt[t] = cnt[t];
+  const uint32_t total = block_exclusive_scan_lds<kBinBlock>(cnt, ntiles, s_wsum, &s_carry);
+  if (tid == 0) s_base = atomicAdd(j.cursor, total);  // past the room for some: the sum stays below 2^32
+  __syncthreads();
+  const uint32_t base = s_base;
+  const bool fits = total <= j.cap && base <= j.cap - total;
+  if (tid == 0) j.gcnt[blockIdx.x] = fits ? total : 0u;
+  if (fits)
+    for (int t = tid; t < ntiles; t += kBinBlock) chunk_off[t] = base + cnt[t];
+  __syncthreads();
+  for (long b = f0; b < f1; b += round) {
+    const long f = mine(b);
+    WireRec r;
+    r.c = make_float4(0.0f, __int_as_float(0), __int_as_float(-1), 0.0f);
+    if (f < f1) r = j.recs[f];  // this lane's own store
+    const bool list = __float_as_int(r.c.z) >= __float_as_int(r.c.y);
+    if (fits) {
+      if (list) wire_tiles(j, r, [&](int t) { j.entries[base + atomicAdd(&cnt[t], 1u)] = (uint32_t)f; });
+    } else {
+      WSetup s;
+      s.ax = r.a.x; s.ay = r.a.y; s.kx = r.a.z; s.ky = r.a.w;
+      s.ws0 = r.b.x; s.ws1 = r.b.y; s.Az = r.b.z; s.Bz = r.b.w;
+      s.siz = __float_as_int(r.c.x);
+      s.i0 = __float_as_int(r.c.y);
+      draw(s, list ? (uint64_t)((int64_t)__float_as_int(r.c.z) - s.i0 + 1) : 0, f);
+    }
+  }
+}
+
+constexpr int kWireQueue = 128;
+
+// Tile b's wires against its keys in LDS: 64 entries a wave at a time, their steps
+// in the tile laid end to end, a step a lane (the lane's wire from a ballot of the
+// places where entries end, as in tile_body).  A step whose depth is certainly
+// behind the key it would meet is dropped; the others are queued and worked out as
+// the reference does in full waves.
+template <int BLOCK>
+__global__ void __launch_bounds__(BLOCK) k_wire_tile(const WireJob jv) {
+  TINA_KERNARG_JOB(WireJob, j, jv);
+  if (blockIdx.x == 0 && threadIdx.x == 0) j.cursor[0] = 0u;  // every group has reserved its entries
+  extern __shared__ uint32_t pre[];  // [ngroups + 1] entries of the tile before each group's
+  __shared__ unsigned long long tk[kWireTile * kWireTile];
+  __shared__ float4 R0[BLOCK], R1[BLOCK], R2[BLOCK], R3[BLOCK];
+  __shared__ int Mark[BLOCK];
+  __shared__ uint32_t Q[BLOCK / 64][kWireQueue];  // per wave: up to 127 steps (slot | pixel) and their numbers
+  __shared__ int Qi[BLOCK / 64][kWireQueue];
+  __shared__ uint32_t s_wsum[BLOCK / 64], s_carry, s_next;
+  __shared__ int s_tile;
+  const int tid = threadIdx.x, lane = tid & 63, wbase = tid & ~63;
+  const int ntiles = j.ntiles, ngroups = j.ngroups;
+  const Cam& cam = j.cam;
+  const float bx = cam.bias[0], by = cam.bias[1];
+  bool any = false;
+  for (int c = tid; c < ngroups; c += BLOCK) any |= j.gcnt[c] != 0u;
+  if (!__syncthreads_or(any)) return;  // every group has drawn its wires
+  uint32_t* const q = Q[tid >> 6];
+  int* const qi = Qi[tid >> 6];
+  int tag = 0;  // windows walked: each has a tag of its own
+  Mark[tid] = -1;
+  for (;;) {
+    if (tid == 0) s_tile = (int)atomicAdd(&j.cursor[1], 1u);
+    __syncthreads();
+    const int t = s_tile;
+    if (t >= ntiles) return;
+    const int ox = (t % j.tiles_x) << kWireTileLog, oy = (t / j.tiles_x) << kWireTileLog;
+    const int tw = min(kWireTile, cam.W - ox), th = min(kWireTile, cam.H - oy);
+    const uint32_t total = block_exclusive_scan<BLOCK>(
+        ngroups, [&](int c) { return j.gcnt[c] ? j.chunk_cnt[(size_t)c * ntiles + t] : 0u; }, [&](int c, uint32_t o) { pre[c] = o; }, s_wsum,
+        &s_carry);
+    if (total == 0) continue;
+    if (tid == 0) {
+      pre[ngroups] = total;
+      s_next = 0;
+    }
+    for (int i = tid; i < kWireTile * kWireTile; i += BLOCK) {
+      const int lx = i & (kWireTile - 1), ly = i >> kWireTileLog;
+      if (lx < tw && ly < th) tk[i] = j.keys[(size_t)(oy + ly) * cam.W + ox + lx];
+    }
+    __syncthreads();
+    const float fox = (float)ox, foy = (float)oy, ftw = (float)tw, fth = (float)th;
+    for (;;) {
+      uint32_t b0 = 0;
+      if (lane == 0) b0 = atomicAdd(&s_next, 64u);
+      b0 = __shfl(b0, 0, 64);
+      if (b0 >= total) break;
+      const uint32_t v = b0 + lane;
+      int cnt = 0;
+      WireRec r;
+      uint32_t id = 0;
+      int s0 = 0;
+      if (v < total) {
+        int lo = 0, hi = ngroups;  // pre[lo] <= v < pre[hi]
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (pre[mid] <= v) lo = mid; else hi = mid;
+        }
+        const uint32_t f = j.entries[j.chunk_off[(size_t)lo * ntiles + t] + (v - pre[lo])];
+        r = j.recs[f];
+        id = j.id_base + f;
+        const int siz = __float_as_int(r.c.x);
+        double l = __float_as_int(r.c.y), h = __float_as_int(r.c.z);
+        wire_clip((double)r.a.x + (double)bx, r.a.z, ox, ox + tw, wire_axis_err(r.a.x, r.a.z, siz, bx), l, h);
+        wire_clip((double)r.a.y + (double)by, r.a.w, oy, oy + th, wire_axis_err(r.a.y, r.a.w, siz, by), l, h);
+        if (l <= h) {
+          s0 = (int)ceil(fmax(l - 0.01, (double)__float_as_int(r.c.y)));
+          cnt = ((int)floor(fmin(h + 0.01, (double)__float_as_int(r.c.z))) - s0 + 2) >> 1;  // pairs of steps
+        }
+      }
+      const unsigned long long live = __ballot(cnt > 0);
+      const int end = wave_inclusive_scan(cnt > 0 ? cnt : 0, lane);
+      const int wtotal = __shfl(end, 63, 64);
+      if (cnt > 0) {
+        const int slot = wbase + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(live >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)live, 0u));
+        R0[slot] = r.a;
+        R1[slot] = r.b;
+        R2[slot] = make_float4(r.c.x, __int_as_float(s0 - 2 * (end - cnt)), __uint_as_float(id), r.c.w);
+        R3[slot] = r.d;
+      }
+      wave_sync_lds();
+      int qn = 0;     // uniform: pending steps in the queue
+      int kbase = 0;  // uniform: entries whose steps all precede the window
+      auto exact = [&](int e) {  // queue entry e: its depth as wire_step has it, into the tile
+        const uint32_t code = q[e];
+        const int k = wbase + (int)(code >> (2 * kWireTileLog));
+        const float4 w = R1[k], c = R2[k];
+        const float cor = fdiv_rn((float)qi[e], (float)__float_as_int(c.x));
+        float w0 = (1.0f - cor) * w.x, w1 = cor * w.y;
+        const RcpRN R = rcp_rn(w0 + w1);
+        w0 = div_rn(w0, R);
+        w1 = div_rn(w1, R);
+        const int32_t depth = f2i_sat(((w0 * w.z) + (w1 * w.w)) * (float)TINA_MAXDEPTH);
+        atomicMin(&tk[code & (kWireTile * kWireTile - 1)], (unsigned long long)pack_key(depth, __float_as_uint(c.z)));
+      };
+      for (int g0 = 0; g0 < wtotal; g0 += 64) {
+        tag++;
+        if (cnt > 0 && end - 1 >= g0 && end - 1 < g0 + 64) Mark[wbase + end - 1 - g0] = tag;
+        wave_sync_lds();
+        const unsigned long long ends = __ballot(Mark[tid] == tag);
+        const int g = g0 + lane;
+        bool keep[2] = {false, false};
+        uint32_t code[2] = {0u, 0u};
+        int i = 0;
+        if (g < wtotal) {
+          const int k = kbase + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(ends >> 32),
+                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)ends, 0u));
+          const float4 a = R0[wbase + k], c = R2[wbase + k], d = R3[wbase + k];
+          i = __float_as_int(c.y) + 2 * g;
+          // steps i and i + 1: the latter may lie past the entry's range, where it is
+          // a step of the wire all the same (or none, past siz)
+  #pragma unroll
+          for (int p = 0; p < 2; p++) {
+            const float fi = (float)(i + p);
+            // the pixel as wire_step has it, less the tile's corner (exact where it matters)
+            const float X = floorf((a.x + a.z * fi) + bx) - fox, Y = floorf((a.y + a.w * fi) + by) - foy;
+            if ((X >= 0.0f) & (X < ftw) & (Y >= 0.0f) & (Y < fth) & (i + p <= __float_as_int(c.x))) {
+              const int at = ((int)Y << kWireTileLog) | (int)X;
+              const uint32_t kh = ((const volatile uint32_t*)tk)[2 * at + 1];
+              const float kd = (float)(int32_t)(kh ^ 0x80000000u) * 0x1p-30f;
+              const float zn = __builtin_fmaf(d.y, fi, d.x), zd = __builtin_fmaf(d.w, fi, d.z);
+              keep[p] = !(zn - kd * zd > c.w);
+              code[p] = ((uint32_t)k << (2 * kWireTileLog)) | (uint32_t)at;
+            }
+          }
+        }
+        kbase += __popcll(ends);
+  #pragma unroll
+        for (int p = 0; p < 2; p++) {
+          const unsigned long long m = __ballot(keep[p]);
+          if (keep[p]) {
+            const int at = qn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            q[at] = code[p];
+            qi[at] = i + p;
+          }
+          qn += __popcll(m);
+          wave_sync_lds();
+          if (qn >= 64) {  // a full wave of them; the rest (at most 63) moves down
+            exact(lane);
+            const int rest = qn - 64;
+            const uint32_t mc = lane < rest ? q[64 + lane] : 0u;
+            const int mi = lane < rest ? qi[64 + lane] : 0;
+            wave_sync_lds();
+            if (lane < rest) {
+              q[lane] = mc;
+              qi[lane] = mi;
+            }
+            qn = rest;
+            wave_sync_lds();
+          }
+        }
+      }
+      if (lane < qn) exact(lane);
+      wave_sync_lds();
+    }
+    __syncthreads();
+    for (int i = tid; i < kWireTile * kWireTile; i += BLOCK) {
+      const int lx = i & (kWireTile - 1), ly = i >> kWireTileLog;
+      if (lx < tw && ly < th) j.keys[(size_t)(oy + ly) * cam.W + ox + lx] = tk[i];
+    }
+    __syncthreads();
+  }
+}
+
+// Lanes of a tile's workgroup: 512 while the tiles are several rounds of workgroups
+// (256: 414 us against 318 for 200 k wires of 600 px, whose fullest tiles finish
+// last), 1,024 on small screens (50 k such wires at 512 x 512: 110 us, 512 lanes 146).
+inline int wire_tile_block(int ntiles, int ncu) { return ntiles >= 4 * ncu ? 512 : 1024; }
+
+inline void launch_wire_tile(const WireJob& j, int ncu, hipStream_t s) {
+  const int grid = std::min(j.ntiles, 2 * ncu);  // each takes the next tile until none is left
+  const size_t lds = (size_t)(j.ngroups + 1) * 4;
+  if (wire_tile_block(j.ntiles, ncu) == 512)
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wire_tile<512>), dim3(grid), dim3(512), lds, s, j);
+  else
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wire_tile<1024>), dim3(grid), dim3(1024), lds, s, j);
 }
 
 // Pixels won by ids [id_base, id_base + n) take color; with bg_on, empty pixels take bg.

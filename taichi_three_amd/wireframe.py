@@ -61,6 +61,7 @@ class WireframeRaster:
         self._fb = fb
         self._mesh = mesh
         self.nfaces = n
+        self.engine.reserve_wires(n)
         self.id_base = self.engine._id_cursor
         self.engine._id_cursor += n
 
@@ -72,6 +73,7 @@ class WireframeRaster:
         if self._mesh is self._own and self._fb is not None:
             self._fb = self._own.face_buffers()
             self.nfaces = int(self._fb['nfaces'])
+            self.engine.reserve_wires(self.nfaces)
             self.engine._id_cursor = max(self.engine._id_cursor, self.id_base + self.nfaces)
         else:
             self.set_object(self._own)
