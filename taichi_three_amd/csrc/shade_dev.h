@@ -492,8 +492,8 @@ __device__ __forceinline__ V3 view_ray(const Cam& cam, int px, int py) {
 // For these the kernel is compiled with the program fixed, so no parameter
 // array and no interpreter stack are needed; the arithmetic (and its order) is
 // the one run_material performs for the same program.
-// PROG_PARTICLE is the generic program over particle fragments.
-enum Prog { PROG_GENERIC = 0, PROG_DIFFUSE = 1, PROG_CLASSIC = 2, PROG_BLINN = 3, PROG_PBR = 4, PROG_PARTICLE = 5 };
+// PAR: the fragments are a particle's instead of a face's.
+enum Prog { PROG_GENERIC = 0, PROG_DIFFUSE = 1, PROG_CLASSIC = 2, PROG_BLINN = 3, PROG_PBR = 4 };
 
 // Value of a non-derived parameter slot (everything but FRESNEL and TEXTURE).
 __device__ __forceinline__ V3 eval_basic(const tina_param& p, uint32_t f, const Frag& fr) {
@@ -606,14 +606,14 @@ __device__ __forceinline__ V3 shade_core(const ShadeArgs& a, V3 n, V3 pos, V3 V,
   return res;
 }
 
-template <int PROG, bool IBL>
+template <int PROG, bool IBL, bool PAR = false>
 __device__ __forceinline__ V3 shade_pixel(const ShadeArgs& a, uint32_t f, int px, int py) {
   Frag fr;
-  if constexpr (PROG == PROG_PARTICLE) particle_fragment(a, f, px, py, fr);
+  if constexpr (PAR) particle_fragment(a, f, px, py, fr);
   else fragment(a, f, px, py, fr);
   const V3 viewdir = vneg(view_ray(a.cam, px, py));
   V3 res;
-  if constexpr (PROG == PROG_GENERIC || PROG == PROG_PARTICLE) {
+  if constexpr (PROG == PROG_GENERIC) {
     Slots pv;
     eval_params(a.mat, f, fr.pos, fr.nrm, fr.tc, fr.color, pv);
     res = lighting(a.mat, pv, a.lights, a.ibl, IBL ? (a.flags | TINA_IBL) : (a.flags & ~TINA_IBL), fr.pos,

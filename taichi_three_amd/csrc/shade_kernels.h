@@ -1,6 +1,6 @@
 // shade_kernels.h -- deferred shading and the image passes.
 //
-//   k_shade<PROG, IBL>  render_color + Shader + Lighting + material (+ ACES, + bg)
+//   k_shade<PROG, IBL, PAR>  render_color + Shader + Lighting + material (+ ACES, + bg)
 //                       (tina/core/triangle.py:133-153, shader.py:112-131,
 //                       lighting.py:84-98): each workgroup owns a chunk of pixels;
 //                       it reads their keys, paints the empty ones with the
@@ -33,7 +33,7 @@ __device__ __forceinline__ void store_rgb(float* __restrict__ img, long P, V3 c)
 
 // Pixels [chunk * PIX, (chunk + 1) * PIX) of one shade call (the body of k_shade
 // and k_bshade).
-template <int PROG, bool IBL, int PIX>
+template <int PROG, bool IBL, bool PAR, int PIX>
 __device__ __forceinline__ void shade_chunk(const ShadeArgs& a, const uint64_t* __restrict__ keys,
                                             float* __restrict__ img, long chunk) {
   static_assert(PIX % kBlock == 0, "whole rows of the workgroup");
@@ -77,11 +77,11 @@ __device__ __forceinline__ void shade_chunk(const ShadeArgs& a, const uint64_t* 
   for (uint32_t j = tid; j < n; j += kBlock) {
     const long P = base + s_pix[j];
     const int px = (int)(P % a.cam.W), py = (int)(P / a.cam.W);
-    store_rgb(img, P, shade_pixel<PROG, IBL>(a, s_face[j], px, py));
+    store_rgb(img, P, shade_pixel<PROG, IBL, PAR>(a, s_face[j], px, py));
   }
 }
 
-template <int PROG, bool IBL>
+template <int PROG, bool IBL, bool PAR>
 __global__ void __launch_bounds__(kBlock)
 k_shade(const ShadeArgs a_by_value, const uint64_t* __restrict__ keys, float* __restrict__ img) {
   // Read the 2 KB argument block in place (it is the first kernel argument, at
@@ -93,15 +93,21 @@ k_shade(const ShadeArgs a_by_value, const uint64_t* __restrict__ keys, float* __
 #else
   const ShadeArgs& a = a_by_value;  // the host pass only needs the signature
 #endif
-  shade_chunk<PROG, IBL, kShadePix>(a, keys, img, blockIdx.x);
+  shade_chunk<PROG, IBL, PAR, kShadePix>(a, keys, img, blockIdx.x);
 }
 
 // The same pass held to eight waves per SIMD, for the fixed programs without
-// IBL: they fit 64 VGPRs with no spills once the compiler is asked to (78
+// IBL: faces fit 64 VGPRs with hardly a spill once the compiler is asked to (78
 // SGPRs instead of 106, which held seven waves); the 1080p/2M PBR shade takes
-// 55.5 us instead of 57.8.  The IBL, generic and particle programs would spill
-// at that budget and keep k_shade.
-template <int PROG>
+// 55.5 us instead of 57.8.  Particles (PAR) spill 44 bytes under Classic and
+// Blinn and run the same at either budget (1 M particles at 1080p, frame 172.9 us
+// against 171.7).  The IBL and generic programs would spill at that budget and
+// keep k_shade.
+// A particle fragment is bound by the interpreter when the program is generic: its
+// 300 bytes of parameters and stack a lane live in scratch.  The fixed programs took
+// that frame from 194.5 to 159.8 us (Diffuse), 223 to 168 (PBR), and with a sky
+// from 370 to 234 (PBR) and 299 to 175 (Diffuse).
+template <int PROG, bool PAR>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8)))
 k_shade8(const ShadeArgs a_by_value, const uint64_t* __restrict__ keys, float* __restrict__ img) {
   (void)a_by_value;
@@ -110,7 +116,7 @@ k_shade8(const ShadeArgs a_by_value, const uint64_t* __restrict__ keys, float* _
 #else
   const ShadeArgs& a = a_by_value;
 #endif
-  shade_chunk<PROG, false, kShadePix>(a, keys, img, blockIdx.x);
+  shade_chunk<PROG, false, PAR, kShadePix>(a, keys, img, blockIdx.x);
 }
 
 // One scene of a batched shade: its arguments, key buffer and image.
@@ -133,36 +139,35 @@ k_bshade(const BatchShade* __restrict__ scenes, const int* __restrict__ prefix, 
       if (prefix[mid] <= item) lo = mid; else hi = mid;
     }
     const BatchShade& sc = scenes[lo];
-    shade_chunk<PROG, IBL, kBatchShadePix>(sc.a, sc.keys, sc.img, item - prefix[lo]);
+    shade_chunk<PROG, IBL, false, kBatchShadePix>(sc.a, sc.keys, sc.img, item - prefix[lo]);
     __syncthreads();
   }
 }
 
-template <int PROG, bool IBL>
+template <int PROG, bool IBL, bool PAR>
 void launch_shade(unsigned grid, hipStream_t s, const ShadeArgs& a, const uint64_t* keys, float* img) {
-  if constexpr (!IBL && PROG != PROG_GENERIC && PROG != PROG_PARTICLE)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_shade8<PROG>), dim3(grid), dim3(kBlock), 0, s, a, keys, img);
+  if constexpr (!IBL && PROG != PROG_GENERIC)
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_shade8<PROG, PAR>), dim3(grid), dim3(kBlock), 0, s, a, keys, img);
   else
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_shade<PROG, IBL>), dim3(grid), dim3(kBlock), 0, s, a, keys, img);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_shade<PROG, IBL, PAR>), dim3(grid), dim3(kBlock), 0, s, a, keys, img);
 }
 
-inline void dispatch_shade(int prog, bool ibl, unsigned grid, hipStream_t s, const ShadeArgs& a,
-                           const uint64_t* keys, float* img) {
+template <bool PAR>
+void dispatch_shade(int prog, bool ibl, unsigned grid, hipStream_t s, const ShadeArgs& a, const uint64_t* keys,
+                    float* img) {
   if (ibl) {
     switch (prog) {
-      case PROG_DIFFUSE: launch_shade<PROG_DIFFUSE, true>(grid, s, a, keys, img); break;
-      case PROG_PBR: launch_shade<PROG_PBR, true>(grid, s, a, keys, img); break;
-      case PROG_PARTICLE: launch_shade<PROG_PARTICLE, true>(grid, s, a, keys, img); break;
-      default: launch_shade<PROG_GENERIC, true>(grid, s, a, keys, img); break;
+      case PROG_DIFFUSE: launch_shade<PROG_DIFFUSE, true, PAR>(grid, s, a, keys, img); break;
+      case PROG_PBR: launch_shade<PROG_PBR, true, PAR>(grid, s, a, keys, img); break;
+      default: launch_shade<PROG_GENERIC, true, PAR>(grid, s, a, keys, img); break;
     }
   } else {
     switch (prog) {
-      case PROG_DIFFUSE: launch_shade<PROG_DIFFUSE, false>(grid, s, a, keys, img); break;
-      case PROG_CLASSIC: launch_shade<PROG_CLASSIC, false>(grid, s, a, keys, img); break;
-      case PROG_BLINN: launch_shade<PROG_BLINN, false>(grid, s, a, keys, img); break;
-      case PROG_PBR: launch_shade<PROG_PBR, false>(grid, s, a, keys, img); break;
-      case PROG_PARTICLE: launch_shade<PROG_PARTICLE, false>(grid, s, a, keys, img); break;
-      default: launch_shade<PROG_GENERIC, false>(grid, s, a, keys, img); break;
+      case PROG_DIFFUSE: launch_shade<PROG_DIFFUSE, false, PAR>(grid, s, a, keys, img); break;
+      case PROG_CLASSIC: launch_shade<PROG_CLASSIC, false, PAR>(grid, s, a, keys, img); break;
+      case PROG_BLINN: launch_shade<PROG_BLINN, false, PAR>(grid, s, a, keys, img); break;
+      case PROG_PBR: launch_shade<PROG_PBR, false, PAR>(grid, s, a, keys, img); break;
+      default: launch_shade<PROG_GENERIC, false, PAR>(grid, s, a, keys, img); break;
     }
   }
 }

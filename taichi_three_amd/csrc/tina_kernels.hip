@@ -730,9 +730,9 @@ int tina_shade(tina_ctx* c, const tina_mesh* mesh, const tina_material* mat, con
   if ((rc = flush_clear(c, (hipStream_t)stream))) return rc;
   const long npix = (long)c->W * c->H;
   const bool ibl_mode = (flags & TINA_IBL) != 0;
-  const int prog = (flags & TINA_PARTICLES) ? (int)PROG_PARTICLE : classify_program(a.mat, ibl_mode);
-  dispatch_shade(prog, ibl_mode, grid_for(npix, kShadePix, 0x7fffffff),
-                 (hipStream_t)stream, a, c->keys, d_img);
+  const int prog = classify_program(a.mat, ibl_mode);
+  (flags & TINA_PARTICLES ? dispatch_shade<true> : dispatch_shade<false>)(
+      prog, ibl_mode, grid_for(npix, kShadePix, 0x7fffffff), (hipStream_t)stream, a, c->keys, d_img);
   TINA_LAUNCH(c, "k_shade");
   return TINA_OK;
 }
