@@ -102,83 +102,149 @@ k_bloom_blur(const float* __restrict__ src, float* __restrict__ dst, int hw, int
   }
 }
 
-// The same blur with the taps read from LDS.  Along x a workgroup stages 256
-// pixels of one row plus `radius` on each side; along y it stages a tile of TX
-// columns by 32 rows plus `radius` rows above and below (TX = 32 or 16, chosen
-// so the tile fits 64 KB).  Staged texels are the clamped ones the direct
-// kernel reads, kept as three planes (no bank conflicts), and every output sums
-// its taps in the same order: identical results, one HBM/L2 read per staged
-// texel instead of 2 radius + 1 per output.
-constexpr int kBlurRow = 256;
-constexpr int kBlurRows = 32;
+// The same blur with the taps read from LDS, R consecutive outputs a lane: the
+// inputs k before and k after them are two windows of R registers that move by one
+// a tap, so a tap costs a lane two LDS reads and 3 R operations instead of 2 R reads.
+// Every output sums its taps in the same order: identical results.
+//   along x  a wave per channel of 64 R pixels of one row, staged as three planes
+//            with a word of padding each R (lanes R apart fall on different banks)
+//   along y  a lane per float of the row (3 hw of them), 64 to a workgroup, a wave
+//            per R rows
+// Bound by VALU issue (three operations a tap and output, 8 us a pass at 1080p with
+// its radius of 67); one output a lane was bound by LDS reads.  1080p, radius 67:
+// 21 -> 14 us along x, 26 -> 14 along y (R = 8 along x 18); the whole bloom 65 -> 47,
+// at radius 150 102 -> 72, at 200 (unstaged along y before) 185 -> 84.
+constexpr int kBlurX = 4, kBlurXSeg = 64 * kBlurX;                  // R along x, pixels a workgroup
+constexpr int kBlurY = 4, kBlurYWaves = 8, kBlurYRows = kBlurY * kBlurYWaves;  // R along y, rows a workgroup
+constexpr size_t kBlurLds = 150 * 1024;
 
-__global__ void __launch_bounds__(kBlock)
-k_bloom_blur_x(const float* __restrict__ src, float* __restrict__ dst, int hw, int hh, const float* __restrict__ gwei,
-               int radius) {
-  extern __shared__ uint32_t lds_words[];
-  float* lds = (float*)lds_words;
-  const int n = kBlurRow + 2 * radius;
-  const int y = blockIdx.y, x0 = blockIdx.x * kBlurRow, t = threadIdx.x;
-  for (int i = t; i < n; i += kBlock) {
-    const int xs = min(max(x0 - radius + i, 0), hw - 1);
-    const float* p = src + ((long)y * hw + xs) * 3;
-    lds[i] = p[0];
-    lds[n + i] = p[1];
-    lds[2 * n + i] = p[2];
-  }
-  __syncthreads();
-  const int x = x0 + t;
-  if (x >= hw) return;
-  const int i = t + radius;
+inline size_t blur_margin(int radius, int R) { return ((size_t)radius + R - 1) / R; }  // groups of R on each side
+inline size_t blur_x_lds(int radius) { return (64 + 2 * blur_margin(radius, kBlurX)) * (kBlurX + 1) * 12; }
+inline size_t blur_y_lds(int radius) { return (kBlurYWaves + 2 * blur_margin(radius, kBlurY)) * kBlurY * 64 * 4; }
+
+// The taps 1..radius of R outputs whose inputs are win: left(k, v) and right(k, v)
+// give the inputs that enter the windows at taps k + 1 .. k + R, k a multiple of R.
+template <int R, class Left, class Right>
+__device__ __forceinline__ void blur_taps(const float* __restrict__ gwei, int radius, const float (&win)[R], float (&acc)[R],
+                                          Left&& left, Right&& right) {
+  float lo[R], hi[R];
   const float g0 = gwei[0];
-  V3 res = v3(lds[i] * g0, lds[n + i] * g0, lds[2 * n + i] * g0);
-  for (int k = 1; k <= radius; k++) {
-    const V3 val = v3(lds[i - k] + lds[i + k], lds[n + i - k] + lds[n + i + k], lds[2 * n + i - k] + lds[2 * n + i + k]);
-    const float g = gwei[k];
-    res = vadd(res, v3(val.x * g, val.y * g, val.z * g));
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    lo[r] = hi[r] = win[r];
+    acc[r] = win[r] * g0;
   }
-  float* o = dst + ((long)y * hw + x) * 3;
-  o[0] = res.x;
-  o[1] = res.y;
-  o[2] = res.z;
+  auto tap = [&](float l, float h, float g) {
+#pragma unroll
+    for (int r = R - 1; r > 0; r--) lo[r] = lo[r - 1];
+    lo[0] = l;
+#pragma unroll
+    for (int r = 0; r < R - 1; r++) hi[r] = hi[r + 1];
+    hi[R - 1] = h;
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = acc[r] + (lo[r] + hi[r]) * g;
+  };
+  int k = 0;
+  float nl[R], nr[R];
+  for (; k + R <= radius; k += R) {  // no branch between the taps: their reads go out together
+    left(k, nl);
+    right(k, nr);
+#pragma unroll
+    for (int u = 0; u < R; u++) tap(nl[u], nr[u], gwei[k + 1 + u]);
+  }
+  if (k == radius) return;
+  left(k, nl);
+  right(k, nr);
+#pragma unroll
+  for (int u = 0; u < R - 1; u++)
+    if (k + u < radius) tap(nl[u], nr[u], gwei[k + 1 + u]);
 }
 
-template <int TX>
-__global__ void __launch_bounds__(kBlock)
-k_bloom_blur_y(const float* __restrict__ src, float* __restrict__ dst, int hw, int hh, const float* __restrict__ gwei,
+__global__ void __launch_bounds__(192)
+k_bloom_blur_x(const float* __restrict__ src, float* __restrict__ dst, int hw, int hh, const float* __restrict__ gwei,
                int radius) {
+  constexpr int R = kBlurX, P = R + 1;
   extern __shared__ uint32_t lds_words[];
-  float* lds = (float*)lds_words;
-  const int rows = kBlurRows + 2 * radius, n = rows * TX;
-  const int x0 = blockIdx.x * TX, y0 = blockIdx.y * kBlurRows, t = threadIdx.x;
-  for (int idx = t; idx < n; idx += kBlock) {
-    const int r = idx / TX, c = idx - r * TX;
-    const int xs = min(x0 + c, hw - 1), ys = min(max(y0 - radius + r, 0), hh - 1);
-    const float* p = src + ((long)ys * hw + xs) * 3;
-    lds[idx] = p[0];
-    lds[n + idx] = p[1];
-    lds[2 * n + idx] = p[2];
+  float* const lds = (float*)lds_words;
+  const int margin = (radius + R - 1) / R;  // in groups of R pixels
+  const int n = kBlurXSeg + 2 * margin * R, plane = n / R * P;
+  const int y = blockIdx.y, x0 = blockIdx.x * kBlurXSeg, t = threadIdx.x;
+  for (int i0 = t; i0 < n; i0 += 2 * 192) {
+    V3 v[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) v[u] = ld_px(src, hw, min(max(x0 - margin * R + i0 + 192 * u, 0), hw - 1), y);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int i = i0 + 192 * u, at = i + i / R;
+      if (i >= n) break;
+      lds[at] = v[u].x;
+      lds[plane + at] = v[u].y;
+      lds[2 * plane + at] = v[u].z;
+    }
   }
   __syncthreads();
-  const int c = t % TX, x = x0 + c;
+  const int c = t >> 6, x = x0 + (t & 63) * R;
   if (x >= hw) return;
-  const float g0 = gwei[0];
-  for (int ry = t / TX; ry < kBlurRows; ry += kBlock / TX) {
-    const int y = y0 + ry;
-    if (y >= hh) break;
-    const int i = (ry + radius) * TX + c;
-    V3 res = v3(lds[i] * g0, lds[n + i] * g0, lds[2 * n + i] * g0);
-    for (int k = 1; k <= radius; k++) {
-      const int a = i - k * TX, b = i + k * TX;
-      const V3 val = v3(lds[a] + lds[b], lds[n + a] + lds[n + b], lds[2 * n + a] + lds[2 * n + b]);
-      const float g = gwei[k];
-      res = vadd(res, v3(val.x * g, val.y * g, val.z * g));
-    }
-    float* o = dst + ((long)y * hw + x) * 3;
-    o[0] = res.x;
-    o[1] = res.y;
-    o[2] = res.z;
+  const float* const w = lds + c * plane + ((t & 63) + margin) * P;  // this lane's outputs
+  float win[R], acc[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) win[r] = w[r];
+  blur_taps<R>(
+      gwei, radius, win, acc,
+      [&](int k, float (&v)[R]) {
+        const float* const q = w - (k / R + 1) * P;
+#pragma unroll
+        for (int u = 0; u < R; u++) v[u] = q[R - 1 - u];
+      },
+      [&](int k, float (&v)[R]) {
+        const float* const q = w + (k / R + 1) * P;
+#pragma unroll
+        for (int u = 0; u < R; u++) v[u] = q[u];
+      });
+  float* o = dst + ((long)y * hw + x) * 3 + c;
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if (x + r < hw) o[3 * r] = acc[r];
+}
+
+__global__ void __launch_bounds__(64 * kBlurYWaves)
+k_bloom_blur_y(const float* __restrict__ src, float* __restrict__ dst, int hw, int hh, const float* __restrict__ gwei,
+               int radius) {
+  constexpr int R = kBlurY;
+  extern __shared__ uint32_t lds_words[];
+  float* const lds = (float*)lds_words;
+  const int margin = (radius + R - 1) / R * R, rows = kBlurYRows + 2 * margin, cols = 3 * hw;
+  const int y0 = blockIdx.y * kBlurYRows, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = blockIdx.x * 64 + lane, cs = min(col, cols - 1);
+  static_assert(2 * R % 8 == 0 && kBlurYRows % 8 == 0, "rows go eight at a time");
+  for (int r0 = 8 * wave; r0 < rows; r0 += 8 * kBlurYWaves) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = src[(long)min(max(y0 - margin + r0 + u, 0), hh - 1) * cols + cs];
+#pragma unroll
+    for (int u = 0; u < 8; u++) lds[(r0 + u) * 64 + lane] = v[u];
   }
+  __syncthreads();
+  const int y = y0 + wave * R;
+  if (col >= cols || y >= hh) return;
+  const float* const w = lds + (wave * R + margin) * 64 + lane;  // this lane's outputs
+  float win[R], acc[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) win[r] = w[r * 64];
+  blur_taps<R>(
+      gwei, radius, win, acc,
+      [&](int k, float (&v)[R]) {
+#pragma unroll
+        for (int u = 0; u < R; u++) v[u] = w[-(k + 1 + u) * 64];
+      },
+      [&](int k, float (&v)[R]) {
+#pragma unroll
+        for (int u = 0; u < R; u++) v[u] = w[(k + R + u) * 64];
+      });
+  float* o = dst + (long)y * cols + col;
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if (y + r < hh) o[(long)r * cols] = acc[r];
 }
 
 // image[I] += bilerp(half, I / 2)

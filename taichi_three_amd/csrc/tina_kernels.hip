@@ -138,6 +138,8 @@ void allow_big_lds() {
   static const bool done = [] {
     (void)hipFuncSetAttribute((const void*)k_bin, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBudget);
     (void)hipFuncSetAttribute((const void*)k_wire_bin, hipFuncAttributeMaxDynamicSharedMemorySize, kWireLds);
+    (void)hipFuncSetAttribute((const void*)k_bloom_blur_x, hipFuncAttributeMaxDynamicSharedMemorySize, kBlurLds);
+    (void)hipFuncSetAttribute((const void*)k_bloom_blur_y, hipFuncAttributeMaxDynamicSharedMemorySize, kBlurLds);
     (void)hipFuncSetAttribute((const void*)k_bbin, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBudget);
     (void)hipGetLastError();
     return true;
@@ -767,22 +769,18 @@ int tina_bloom(float* d_img, int width, int height, float thresh, float factor, 
   const long nh = (long)hw * hh, n = (long)width * height;
   hipLaunchKernelGGL(k_bloom_down, dim3(grid_for(nh, kBlock, 4096)), dim3(kBlock), 0, s, d_img, width, d_half, hw, hh,
                      thresh, scale, factor);
-  // the LDS-staged passes when their tiles fit 64 KB (radius up to ~1300 along x, ~150 along y)
-  const size_t lds_x = (size_t)(kBlurRow + 2 * radius) * 12;
-  const size_t lds_y32 = (size_t)(kBlurRows + 2 * radius) * 32 * 12, lds_y16 = lds_y32 / 2;
-  if (lds_x <= 65536)
-    hipLaunchKernelGGL(k_bloom_blur_x, dim3((hw + kBlurRow - 1) / kBlurRow, hh), dim3(kBlock), lds_x, s, d_half,
-                       d_tmp, hw, hh, d_gwei, radius);
+  // the staged passes where their tiles fit (radius up to ~5000 along x, 280 along y)
+  allow_big_lds();
+  const size_t lds_x = blur_x_lds(radius), lds_y = blur_y_lds(radius);
+  if (lds_x <= kBlurLds)
+    hipLaunchKernelGGL(k_bloom_blur_x, dim3((hw + kBlurXSeg - 1) / kBlurXSeg, hh), dim3(192), lds_x, s, d_half, d_tmp,
+                       hw, hh, d_gwei, radius);
   else
     hipLaunchKernelGGL(k_bloom_blur, dim3(grid_for(nh, kBlock, 4096)), dim3(kBlock), 0, s, d_half, d_tmp, hw, hh,
                        d_gwei, radius, 0);
-  const unsigned gy = (unsigned)((hh + kBlurRows - 1) / kBlurRows);
-  if (lds_y32 <= 65536)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bloom_blur_y<32>), dim3((hw + 31) / 32, gy), dim3(kBlock), lds_y32, s, d_tmp,
-                       d_half, hw, hh, d_gwei, radius);
-  else if (lds_y16 <= 65536)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bloom_blur_y<16>), dim3((hw + 15) / 16, gy), dim3(kBlock), lds_y16, s, d_tmp,
-                       d_half, hw, hh, d_gwei, radius);
+  if (lds_y <= kBlurLds)
+    hipLaunchKernelGGL(k_bloom_blur_y, dim3((3 * hw + 63) / 64, (hh + kBlurYRows - 1) / kBlurYRows),
+                       dim3(64 * kBlurYWaves), lds_y, s, d_tmp, d_half, hw, hh, d_gwei, radius);
   else
     hipLaunchKernelGGL(k_bloom_blur, dim3(grid_for(nh, kBlock, 4096)), dim3(kBlock), 0, s, d_tmp, d_half, hw, hh,
                        d_gwei, radius, 1);
