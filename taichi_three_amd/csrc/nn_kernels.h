@@ -279,6 +279,23 @@ __device__ __forceinline__ void grad_bias(const float* D, float* __restrict__ ou
   if (lane < 8) outB[o] = sb;
 }
 
+// The parameters' places in k_mlp_grad's LDS: as in memory but with W2's, W3's and W4's
+// rows kGradRow floats apart, so that lanes reading 16 rows at one column meet
+// different banks; 64 apart they all met one, and the kernel took 22.4 us instead of
+// 20.0 (16,384 samples; of these the matrix cores are busy for 6).
+constexpr int kLdsW2 = kOffW2, kLdsB2 = kLdsW2 + 64 * kGradRow, kLdsW3 = kLdsB2 + 64, kLdsB3 = kLdsW3 + 64 * kGradRow,
+              kLdsW4 = kLdsB3 + 64, kLdsB4 = kLdsW4 + 4 * kGradRow, kLdsParams = kLdsB4 + 4;
+__device__ __forceinline__ int grad_place(int p) {  // of parameter p
+  auto rows = [&](int at, int off) { return at + (p - off) + (p - off) / kNnHid * (kGradRow - kNnHid); };
+  if (p < kOffW2) return p;
+  if (p < kOffB2) return rows(kLdsW2, kOffW2);
+  if (p < kOffW3) return kLdsB2 + (p - kOffB2);
+  if (p < kOffB3) return rows(kLdsW3, kOffW3);
+  if (p < kOffW4) return kLdsB3 + (p - kOffB3);
+  if (p < kOffB4) return rows(kLdsW4, kOffW4);
+  return kLdsB4 + (p - kOffB4);
+}
+
 constexpr int kGradBlock = 512;  // eight waves: two per SIMD, each with half of a layer's tiles
 static_assert(64 * 16 == 2 * kGradBlock, "the feature and gradient staging takes two passes");
 
@@ -288,7 +305,7 @@ k_mlp_grad(const float* __restrict__ params, const float* __restrict__ X, const 
   __shared__ __attribute__((aligned(16))) float sX[64 * 16];   // [s][16]: features, 12..15 zero
   __shared__ __attribute__((aligned(16))) float sH1[64 * kGradRow], sH2[64 * kGradRow], sH3[64 * kGradRow];
   __shared__ __attribute__((aligned(16))) float sGo[64 * 16];  // [s][16]: output gradients, 4..15 zero
-  __shared__ __attribute__((aligned(16))) float sP[kNnParams];   // the parameters, staged once
+  __shared__ __attribute__((aligned(16))) float sP[kLdsParams];   // the parameters, staged once
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, k = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = w & 3, h2 = 2 * (w >> 2);  // this wave's neuron block and first tile of the other dimension
@@ -312,7 +329,7 @@ k_mlp_grad(const float* __restrict__ params, const float* __restrict__ X, const 
 #pragma unroll
   for (int t = 0; t < kPv; t++) {
     const int e = tid + t * kGradBlock;
-    if (e < kNnParams / 4) ((f32x4*)sP)[e] = pv[t];
+    if (e < kNnParams / 4) *(f32x4*)(sP + grad_place(4 * e)) = pv[t];
   }
 #pragma unroll
   for (int t = 0; t < 2; t++) {
@@ -335,17 +352,17 @@ k_mlp_grad(const float* __restrict__ params, const float* __restrict__ X, const 
   for (int kk = 0; kk < 3; kk++) w1[kk] = params_l[kOffW1 + (16 * m + i) * kNnIn + 4 * kk + k];
 #pragma unroll
   for (int kk = 0; kk < 16; kk++) {
-    w2[kk] = params_l[kOffW2 + (16 * m + i) * kNnHid + 16 * k + kk];
-    w3[kk] = params_l[kOffW3 + (16 * m + i) * kNnHid + 16 * k + kk];
-    w4[kk] = i < kNnOut ? params_l[kOffW4 + i * kNnHid + 16 * k + kk] : 0.0f;
-    w3t[kk] = params_l[kOffW3 + (16 * k + kk) * kNnHid + 16 * m + i];
-    w2t[kk] = params_l[kOffW2 + (16 * k + kk) * kNnHid + 16 * m + i];
+    w2[kk] = params_l[kLdsW2 + (16 * m + i) * kGradRow + 16 * k + kk];
+    w3[kk] = params_l[kLdsW3 + (16 * m + i) * kGradRow + 16 * k + kk];
+    w4[kk] = i < kNnOut ? params_l[kLdsW4 + i * kGradRow + 16 * k + kk] : 0.0f;
+    w3t[kk] = params_l[kLdsW3 + (16 * k + kk) * kGradRow + 16 * m + i];
+    w2t[kk] = params_l[kLdsW2 + (16 * k + kk) * kGradRow + 16 * m + i];
   }
-  w4t[0] = k < 3 ? params_l[kOffW4 + k * kNnHid + 16 * m + i] : 0.0f;  // the colour rows of W4 only
+  w4t[0] = k < 3 ? params_l[kLdsW4 + k * kGradRow + 16 * m + i] : 0.0f;  // the colour rows of W4 only
   const f32x4 bias1 = *(const f32x4*)(params_l + kOffB1 + 16 * m + 4 * k);
-  const f32x4 bias2 = *(const f32x4*)(params_l + kOffB2 + 16 * m + 4 * k);
-  const f32x4 bias3 = *(const f32x4*)(params_l + kOffB3 + 16 * m + 4 * k);
-  const f32x4 bias4 = *(const f32x4*)(params_l + kOffB4);
+  const f32x4 bias2 = *(const f32x4*)(params_l + kLdsB2 + 16 * m + 4 * k);
+  const f32x4 bias3 = *(const f32x4*)(params_l + kLdsB3 + 16 * m + 4 * k);
+  const f32x4 bias4 = *(const f32x4*)(params_l + kLdsB4);
   // forward: layer 1 (K = 12 in the order f = 4 kk + k), layers 2 and 3
   {
     f32x4 a1[2] = {bias1, bias1};
@@ -460,7 +477,9 @@ k_mlp_grad(const float* __restrict__ params, const float* __restrict__ X, const 
 // g = the sum of the `nrows` rows of partial; Adam with bias corrections
 // c1 = 1/(1 - b1^t), c2 = 1/(1 - b2^t) supplied by the host.  A workgroup takes
 // 64 parameters: its kAdamGroups waves sum consecutive runs of the rows, each in
-// row order, and wave 0 adds the runs' sums in order (deterministic).
+// row order, and wave 0 adds the runs' sums in order (deterministic).  Bound by the
+// latency of those reads: 4.0 us over the 256 rows of 16,384 samples with eight of
+// them in flight a lane, 6.3 one after the other.
 constexpr int kAdamGroups = 16;
 
 __global__ void __launch_bounds__(64 * kAdamGroups)
@@ -472,8 +491,17 @@ k_mlp_adam(float* __restrict__ params, float* __restrict__ m1, float* __restrict
   const int p = blockIdx.x * 64 + lane;
   const int per = (nrows + kAdamGroups - 1) / kAdamGroups, r0 = wq * per, r1 = min(nrows, r0 + per);
   float g = 0.0f;
-  if (p < kNnParams)
-    for (int r = r0; r < r1; r++) g += partial[(size_t)r * kNnParams + p];
+  if (p < kNnParams) {
+    int r = r0;
+    for (; r + 8 <= r1; r += 8) {  // eight reads on their way, added in row order
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = partial[(size_t)(r + u) * kNnParams + p];
+#pragma unroll
+      for (int u = 0; u < 8; u++) g += v[u];
+    }
+    for (; r < r1; r++) g += partial[(size_t)r * kNnParams + p];
+  }
   s_sum[wq][lane] = g;
   __syncthreads();
   if (wq != 0 || p >= kNnParams) return;
