@@ -199,8 +199,8 @@ int tina_raster_particles(tina_ctx *ctx, const float *d_pos, const float *d_radi
 int tina_raster_wires(tina_ctx *ctx, const float *d_verts, int n, uint32_t id_base, uint32_t flags,
                       void *stream);
 /* Makes the scratch with which tina_raster_wires takes calls of n wires by screen
- * tiles (65,536 wires and more; fewer need none, and without it, or where the memory
- * is short, they are drawn into the depth|id buffer directly, with the same result).
+ * tiles (65,536 wires and more, 131,072 on screens of up to 524,288 pixels; fewer need
+ * none, and without it, or where the memory is short, they are drawn into the depth|id buffer directly, with the same result).
  * Made once per context, at most 60 MB at 1920 x 1080; nothing is made while stream
  * is capturing.  Call it where the wires are bound, outside the frame. */
 int tina_wires_reserve(tina_ctx *ctx, int n, void *stream);

@@ -521,7 +521,7 @@ int tina_raster_wires(tina_ctx* c, const float* d_verts, int n, uint32_t id_base
   hipStream_t s = (hipStream_t)stream;
   int rc = flush_clear(c, s);
   if (rc) return rc;
-  if (c->wires && wires_by_tile(n)) {
+  if (c->wires && wires_by_tile(n, (long)c->W * c->H)) {
     const WireScratch w = wire_scratch(c->W, c->H, c->ncu);
     WireJob j;
     wire_scratch_at(w, c->wires, j);
@@ -552,7 +552,7 @@ int tina_raster_wires(tina_ctx* c, const float* d_verts, int n, uint32_t id_base
 int tina_wires_reserve(tina_ctx* c, int n, void* stream) {
   if (!c) return fail(nullptr, TINA_ERR_INVALID, "ctx is NULL");
   if (n < 0) return fail(c, TINA_ERR_INVALID, "n must be >= 0");
-  if (c->wires || !wires_by_tile(n)) return TINA_OK;
+  if (c->wires || !wires_by_tile(n, (long)c->W * c->H)) return TINA_OK;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing((hipStream_t)stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();

@@ -207,16 +207,18 @@ inline int wires_per_wave(long n, int ncu) {
 // have drawn their wires.
 constexpr int kWireTileLog = 5, kWireTile = 1 << kWireTileLog;
 
-// Calls of this many wires go by tile where their steps are many (kWireGroupSteps).
-// Frames of 1080p with 66 k wires of 600, 150, 50, 15 and 5 px: 408 -> 177 us, 151 ->
-// 104, 80 -> 81, 45 -> 49, 38 -> 40; with 200 k: 818 -> 325, 279 -> 128, 146 -> 98, 76
-// -> 81, 49 -> 54 (at 800 x 450, a third as long: 360 -> 265, 142 -> 72, 82 -> 89, 43 ->
-// 53).  The steps are counted on the device, so a call of short wires pays the tile
-// pass's empty launch and a raster by k_wire_bin, at half of k_wires's waves.  Below
-// this count short wires are the usual ones and the launch is the same price (16 k of
-// 50 px 39 -> 44).
+// Calls of this many wires go by tile where their steps are many (kWireGroupSteps);
+// of twice as many where the keys fit an XCD's L2.  Frames of 1080p with 66 k wires of
+// 600, 150, 50, 15 and 5 px: 408 -> 177 us, 151 -> 104, 80 -> 81, 45 -> 49, 38 -> 40;
+// with 200 k: 818 -> 325, 279 -> 128, 146 -> 98, 76 -> 81, 49 -> 54.  At 800 x 450, a
+// third as long: 200 k 360 -> 265, 142 -> 72, 82 -> 89, 43 -> 53, but 66 k 196 -> 120,
+// 82 -> 85, 45 -> 49, 39 -> 40.  The steps are counted on the device, so a call of
+// short wires pays the tile pass's empty launch and a raster by k_wire_bin, at half of
+// k_wires's waves.  Below these counts short wires are the usual ones and the launch is
+// the same price (16 k of 50 px at 1080p 39 -> 44).
 constexpr int kWireTiledCall = 65536;
-inline bool wires_by_tile(long n) { return n >= kWireTiledCall; }
+constexpr long kXcdL2 = 4L << 20;
+inline bool wires_by_tile(long n, long npix) { return n >= (npix * 8 > kXcdL2 ? kWireTiledCall : 2 * kWireTiledCall); }
 
 // A wire's set-up, one cache line.
 struct WireRec {

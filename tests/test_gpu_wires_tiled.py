@@ -1,4 +1,4 @@
-"""Wire calls by tile (65,536 wires and more), depth and ids bit for bit against the
+"""Wire calls by tile (65,536 wires and more, twice that on small screens), depth and ids bit for bit against the
 oracle: just below and at the count, long and short wires mixed so that a call takes
 both ways, screens that are no multiple of a tile, more wires than the scratch holds
 at a time, entries that do not fit (those groups are drawn), wires with no length,
@@ -29,9 +29,9 @@ def _draw(W, H, wires, clip=False):
 @pytest.mark.parametrize('W,H,n,reach,clip', [
     (1001, 667, 65531, 0.3, False),    # 65,536 with the five extremes: ragged tiles, long wires
     (1001, 667, 65530, 0.3, False),    # one fewer: drawn into memory
-    (640, 360, 70000, 0.004, True),    # about a pixel each: every group draws
+    (1200, 450, 70000, 0.004, True),   # about a pixel each: every group draws
     (97, 61, 262300, 1.2, False),      # more than the 262,144 that go at a time
-    (16384, 3, 65600, 1.2, False),     # 512 tiles in a row: more entries than there is room for
+    (16384, 3, 131067, 1.2, False),    # the small screen's count; 512 tiles in a row: more entries than there is room for
 ])
 def test_tiled_wires_bit_exact(gpu, W, H, n, reach, clip):
     print(f'case: {n} wires {W}x{H} reach {reach} clip={clip}', flush=True)
@@ -50,8 +50,8 @@ def test_two_tiled_calls_share_the_keys(gpu):
     """Two wire objects of 66,000 and 70,000: half their groups short, half long."""
     import torch
     import taichi_three_amd as tina
-    W, H = 800, 450
-    print('case: two tiled wire objects 800x450', flush=True)
+    W, H = 1000, 700
+    print('case: two tiled wire objects 1000x700', flush=True)
     rng = np.random.default_rng(9)
     sets = []
     for k, n in enumerate((66000, 70000)):
