@@ -533,7 +533,7 @@ int tina_raster_wires(tina_ctx* c, const float* d_verts, int n, uint32_t id_base
       j.verts = d_verts + 6 * (size_t)f0;
       j.n = std::min(n - f0, w.room);
       j.id_base = id_base + (uint32_t)f0;
-      j.per = std::max((j.n + c->ncu - 1) / c->ncu, 64);
+      j.per = wires_per_group(j.n, c->ncu);
       j.ngroups = (j.n + j.per - 1) / j.per;
       hipLaunchKernelGGL(k_wire_bin, dim3(j.ngroups), dim3(kBinBlock), (size_t)j.ntiles * 4, s, j);
       TINA_LAUNCH(c, "k_wire_bin");

@@ -244,7 +244,8 @@ struct WireJob {
 };
 
 // Scratch of wire calls by tile: one allocation, kept by the context once a call's
-// count asks for it.  kWireRoom wires go at a time and have kWireEntries entries each
+// count asks for it.  At most kWireRoom wires go at a time, and no more than a lane's
+// one for each lane of a workgroup on every unit; they have kWireEntries entries each
 // (wires of 600 px have about 22); a table of counts and one of offsets for as many
 // groups as the device has units.  1080p: 46 MB.
 constexpr int kWireLds = kLdsBudget - 16 * 1024;  // for k_wire_bin's counts by tile (its static LDS is 9 KB)
@@ -262,7 +263,7 @@ inline WireScratch wire_scratch(int W, int H, int ncu) {
   if (4 * ntiles > kWireLds) return w;
   w.ntiles = (int)ntiles;
   // the count of all entries, at most a few tile rows and columns a wire, has 32 bits
-  w.room = (int)std::min((long)kWireRoom, 0xFFFFFFFFL / (4L * (w.tiles_x + ntiles / w.tiles_x + 4)));
+  w.room = (int)std::min({(long)kWireRoom, (long)kBinBlock * ncu, 0xFFFFFFFFL / (4L * (w.tiles_x + ntiles / w.tiles_x + 4))});
   auto place = [&](size_t n) {
     const size_t at = w.bytes;
     w.bytes += (n + 255) & ~(size_t)255;
@@ -272,10 +273,14 @@ inline WireScratch wire_scratch(int W, int H, int ncu) {
   w.gcnt = place(4 * (size_t)ncu);
   w.chunk_cnt = place(4 * (size_t)ncu * w.ntiles);
   w.chunk_off = place(4 * (size_t)ncu * w.ntiles);
-  w.entries = place(4 * (size_t)kWireRoom * kWireEntries);
-  w.recs = place(sizeof(WireRec) * (size_t)kWireRoom);
+  w.entries = place(4 * (size_t)w.room * kWireEntries);
+  w.recs = place(sizeof(WireRec) * (size_t)w.room);
   return w;
 }
+
+// Wires a group for n of them, n at most the scratch's room: a group for every unit,
+// 64 wires at least.  Never more than k_wire_bin has lanes.
+inline int wires_per_group(int n, int ncu) { return std::max((n + ncu - 1) / ncu, 64); }
 
 inline void wire_scratch_at(const WireScratch& w, void* base, WireJob& j) {
   char* const b = (char*)base;
@@ -285,7 +290,7 @@ inline void wire_scratch_at(const WireScratch& w, void* base, WireJob& j) {
   j.chunk_off = (uint32_t*)(b + w.chunk_off);
   j.entries = (uint32_t*)(b + w.entries);
   j.recs = (WireRec*)(b + w.recs);
-  j.cap = (uint32_t)(kWireRoom * kWireEntries);
+  j.cap = (uint32_t)w.room * kWireEntries;
   j.tiles_x = w.tiles_x;
   j.ntiles = w.ntiles;
 }
@@ -336,18 +341,17 @@ __device__ __forceinline__ void wire_tiles(const WireJob& j, const WireRec& r, F
   }
 }
 
-// Steps of a round of up to 1,024 wires from which they are listed by tile instead
+// Steps of a group of up to 1,024 wires from which they are listed by tile instead
 // of drawn: about 3 M a call, where the two meet (128 k wires of 50 px, 6.4 M steps:
 // 92 us by tile, 113 in memory; 64 k, 3.2 M: 82 either way; twice the limit leaves
 // 64 k of 150 px at 150 instead of 103).
 constexpr uint64_t kWireGroupSteps = 12288;
 
-// Group blockIdx.x's wires, up to 1,024 at a time (pw by each of the sixteen waves):
-// set up, then, where their steps are many, counted per tile and, once the group is
-// through, listed per tile (as bin_group does for faces); where they are few, drawn
-// into memory, so that the tile pass finds nothing to do.  Wires with no length or a
-// value that is not finite, which have no tiles to find, are drawn, as are all of a
-// group whose entries do not fit.
+// Group blockIdx.x's wires, at most one a lane (pw to each of the sixteen waves): set
+// up, then, where their steps are many, counted per tile and listed per tile (as
+// bin_group does for faces); where they are few, drawn into memory, so that the tile
+// pass finds nothing to do.  Wires with no length or a value that is not finite, which
+// have no tiles to find, are drawn, as are all of a group whose entries do not fit.
 __global__ void __launch_bounds__(kBinBlock) k_wire_bin(const WireJob jv) {
   TINA_KERNARG_JOB(WireJob, j, jv);
   extern __shared__ __align__(16) uint32_t lds[];
@@ -357,62 +361,53 @@ __global__ void __launch_bounds__(kBinBlock) k_wire_bin(const WireJob jv) {
   __shared__ int s_mark[kBinBlock], s_slot[kBinBlock];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wbase = tid & ~63, ntiles = j.ntiles;
   constexpr int kWaves = kBinBlock / 64;
-  const int pw = min(64, (j.per + kWaves - 1) / kWaves);
-  const long f0 = (long)blockIdx.x * j.per, f1 = min((long)j.n, f0 + j.per), round = (long)kWaves * pw;
+  const int pw = (j.per + kWaves - 1) / kWaves;
+  const long f0 = (long)blockIdx.x * j.per, f1 = min((long)j.n, f0 + j.per);
+  const long f = lane < pw ? f0 + wave * pw + lane : f1;  // this lane's wire
   const bool clip = (j.flags & TINA_CLIP) != 0;
   unsigned long long* const keys = (unsigned long long*)j.keys;
-  // this lane's wire of the round at b
-  auto mine = [&](long b) { return lane < pw ? b + wave * pw + lane : f1; };
-  auto draw = [&](const WSetup& s, uint64_t steps, long f) {
+  auto draw = [&](const WSetup& s, uint64_t steps) {
     if (__any(steps > 0)) wires_to_memory(j.cam, s, steps, j.id_base + (uint32_t)f, keys, s_mark + wbase, s_slot + wbase);
   };
   s_mark[tid] = -1;
   if (blockIdx.x == 0 && tid == 0) j.cursor[1] = 0u;  // the tile pass's next tile
-  bool listed = false;  // uniform: some round of the group goes by tile
-  for (long b = f0; b < f1; b += round) {
-    const long f = mine(b);
-    if (tid == 0) s_steps = 0;
-    __syncthreads();
-    WSetup s;
-    s.ax = s.ay = s.kx = s.ky = s.ws0 = s.ws1 = s.Az = s.Bz = 0.0f;
-    s.siz = s.i0 = 0;
-    uint64_t steps = 0;
-    if (f < f1 && !wire_setup(j.cam, (gf32*)j.verts, f, clip, s, steps)) steps = 0;
-    if (steps) atomicAdd(&s_steps, (unsigned long long)steps);
-    __syncthreads();
-    const bool tiled = s_steps >= kWireGroupSteps;
-    if (tiled && !listed) {
-      listed = true;
-      for (int t = tid; t < ntiles; t += kBinBlock) cnt[t] = 0;
-      __syncthreads();
-    }
-    const float sum = ((fabsf(s.ax) + fabsf(s.ay)) + (fabsf(s.kx) + fabsf(s.ky))) +
-                      ((fabsf(s.ws0) + fabsf(s.ws1)) + (fabsf(s.Az) + fabsf(s.Bz)));
-    const bool list = tiled && steps > 0 && s.siz > 0 && sum < 1e9f;
-    WireRec r;
-    if (list) {
-      r.a = make_float4(s.ax, s.ay, s.kx, s.ky);
-      r.b = make_float4(s.ws0, s.ws1, s.Az, s.Bz);
-      // z by steps: n / d with n = ws0 Az (1 - c) + ws1 Bz c, d = ws0 (1 - c) + ws1 c, c = i / siz
-      const float is = 1.0f / (float)s.siz, n0 = s.ws0 * s.Az, d0 = s.ws0;
-      r.d = make_float4(n0, (s.ws1 * s.Bz - n0) * is, d0, (s.ws1 - d0) * is);
-      // e: z d computed so, and the reference's own z, are off by less than e (32 roundings
-      // of the largest terms); both ends in front of the camera, or no bound
-      const float mx = fmaxf(s.ws0, s.ws1), mn = fminf(s.ws0, s.ws1);
-      const float e = 32.0f * 5.9604645e-8f * mx * (1.0f + fmaxf(fabsf(s.Az), fabsf(s.Bz))) * (1.0f + mx / mn);
-      r.c = make_float4(__int_as_float(s.siz), __int_as_float(s.i0),
-                        __int_as_float((int)((int64_t)s.i0 + (int64_t)steps - 1)), mn > 0.0f ? e : INFINITY);
-      wire_tiles(j, r, [&](int t) { atomicAdd(&cnt[t], 1u); });
-      j.recs[f] = r;
-    } else if (f < f1 && (tiled || j.per > round)) {
-      j.recs[f].c = make_float4(0.0f, __int_as_float(0), __int_as_float(-1), 0.0f);  // not listed
-    }
-    draw(s, list ? 0 : steps, f);
-  }
-  if (!listed) {  // the tile pass takes no counts from this group
-    if (tid == 0) j.gcnt[blockIdx.x] = 0u;
+  if (tid == 0) s_steps = 0;
+  __syncthreads();
+  WSetup s;
+  s.ax = s.ay = s.kx = s.ky = s.ws0 = s.ws1 = s.Az = s.Bz = 0.0f;
+  s.siz = s.i0 = 0;
+  uint64_t steps = 0;
+  if (f < f1 && !wire_setup(j.cam, (gf32*)j.verts, f, clip, s, steps)) steps = 0;
+  if (steps) atomicAdd(&s_steps, (unsigned long long)steps);
+  __syncthreads();
+  const bool tiled = s_steps >= kWireGroupSteps;  // uniform
+  if (!tiled) {
+    draw(s, steps);
+    if (tid == 0) j.gcnt[blockIdx.x] = 0u;  // the tile pass takes no counts from this group
     return;
   }
+  for (int t = tid; t < ntiles; t += kBinBlock) cnt[t] = 0;
+  __syncthreads();
+  const float sum = ((fabsf(s.ax) + fabsf(s.ay)) + (fabsf(s.kx) + fabsf(s.ky))) +
+                    ((fabsf(s.ws0) + fabsf(s.ws1)) + (fabsf(s.Az) + fabsf(s.Bz)));
+  const bool list = steps > 0 && s.siz > 0 && sum < 1e9f;
+  WireRec r;
+  if (list) {
+    r.a = make_float4(s.ax, s.ay, s.kx, s.ky);
+    r.b = make_float4(s.ws0, s.ws1, s.Az, s.Bz);
+    // z by steps: n / d with n = ws0 Az (1 - c) + ws1 Bz c, d = ws0 (1 - c) + ws1 c, c = i / siz
+    const float is = 1.0f / (float)s.siz, n0 = s.ws0 * s.Az, d0 = s.ws0;
+    r.d = make_float4(n0, (s.ws1 * s.Bz - n0) * is, d0, (s.ws1 - d0) * is);
+    // e: z d computed so, and the reference's own z, are off by less than e (32 roundings
+    // of the largest terms); both ends in front of the camera, or no bound
+    const float mx = fmaxf(s.ws0, s.ws1), mn = fminf(s.ws0, s.ws1);
+    const float e = 32.0f * 5.9604645e-8f * mx * (1.0f + fmaxf(fabsf(s.Az), fabsf(s.Bz))) * (1.0f + mx / mn);
+    r.c = make_float4(__int_as_float(s.siz), __int_as_float(s.i0),
+                      __int_as_float((int)((int64_t)s.i0 + (int64_t)steps - 1)), mn > 0.0f ? e : INFINITY);
+    wire_tiles(j, r, [&](int t) { atomicAdd(&cnt[t], 1u); });
+    j.recs[f] = r;
+  }
+  draw(s, list ? 0 : steps);
   __syncthreads();
   uint32_t* __restrict__ chunk_cnt = j.chunk_cnt + (size_t)blockIdx.x * ntiles;
   uint32_t* __restrict__ chunk_off = j.chunk_off + (size_t)blockIdx.x * ntiles;
@@ -423,26 +418,13 @@ __global__ void __launch_bounds__(kBinBlock) k_wire_bin(const WireJob jv) {
   const uint32_t base = s_base;
   const bool fits = total <= j.cap && base <= j.cap - total;
   if (tid == 0) j.gcnt[blockIdx.x] = fits ? total : 0u;
-  if (fits)
-    for (int t = tid; t < ntiles; t += kBinBlock) chunk_off[t] = base + cnt[t];
-  __syncthreads();
-  for (long b = f0; b < f1; b += round) {
-    const long f = mine(b);
-    WireRec r;
-    r.c = make_float4(0.0f, __int_as_float(0), __int_as_float(-1), 0.0f);
-    if (f < f1) r = j.recs[f];  // this lane's own store
-    const bool list = __float_as_int(r.c.z) >= __float_as_int(r.c.y);
-    if (fits) {
-      if (list) wire_tiles(j, r, [&](int t) { j.entries[base + atomicAdd(&cnt[t], 1u)] = (uint32_t)f; });
-    } else {
-      WSetup s;
-      s.ax = r.a.x; s.ay = r.a.y; s.kx = r.a.z; s.ky = r.a.w;
-      s.ws0 = r.b.x; s.ws1 = r.b.y; s.Az = r.b.z; s.Bz = r.b.w;
-      s.siz = __float_as_int(r.c.x);
-      s.i0 = __float_as_int(r.c.y);
-      draw(s, list ? (uint64_t)((int64_t)__float_as_int(r.c.z) - s.i0 + 1) : 0, f);
-    }
+  if (!fits) {
+    draw(s, list ? steps : 0);
+    return;
   }
+  for (int t = tid; t < ntiles; t += kBinBlock) chunk_off[t] = base + cnt[t];
+  __syncthreads();
+  if (list) wire_tiles(j, r, [&](int t) { j.entries[base + atomicAdd(&cnt[t], 1u)] = (uint32_t)f; });
 }
 
 constexpr int kWireQueue = 128;
