@@ -262,7 +262,8 @@ inline WireScratch wire_scratch(int W, int H, int ncu) {
   w.bytes = 0;
   if (4 * ntiles > kWireLds) return w;
   w.ntiles = (int)ntiles;
-  // the count of all entries, at most a few tile rows and columns a wire, has 32 bits
+  // the count of all entries has 32 bits: a listed wire has three a tile column or row
+  // of its major axis at most (wire_listed)
   w.room = (int)std::min({(long)kWireRoom, (long)kBinBlock * ncu, 0xFFFFFFFFL / (4L * (w.tiles_x + ntiles / w.tiles_x + 4))});
   auto place = [&](size_t n) {
     const size_t at = w.bytes;
@@ -297,13 +298,23 @@ inline void wire_scratch_at(const WireScratch& w, void* base, WireJob& j) {
 
 // Bound on the distance of the binary32 a + k i + bias of a walked step from its
 // exact value: three roundings of at most the magnitudes involved (2^-24 each).
-__device__ __forceinline__ double wire_axis_err(float a, float k, int siz, float bias) {
+__host__ __device__ __forceinline__ double wire_axis_err(float a, float k, int siz, float bias) {
   return 1e-3 + 1e-6 * (fabs((double)a) + fabs((double)k) * (double)siz + fabs((double)bias));
+}
+
+// A wire goes by tile while that bound is at most a quarter of a tile (an end some 8
+// million pixels away) on both axes: its steps over a tile of the major axis then span
+// 48 + 16 pixels of the other, three tiles.  With no such limit a wire that ends 10^9
+// pixels away was listed in every tile, and on screens beyond 16 k tiles the entries'
+// 32-bit count could wrap.  Such wires are drawn.  False for a NaN.
+constexpr double kWireListErr = kWireTile / 4;
+__host__ __device__ __forceinline__ bool wire_listed(float ax, float ay, float kx, float ky, int siz, float bx, float by) {
+  return wire_axis_err(ax, kx, siz, bx) <= kWireListErr && wire_axis_err(ay, ky, siz, by) <= kWireListErr;
 }
 
 // Narrows the steps [lo, hi] to those whose exact position p0 + k i (p0 = a + bias)
 // lies within err of [q0, q1].
-__device__ __forceinline__ void wire_clip(double p0, double k, double q0, double q1, double err, double& lo, double& hi) {
+__host__ __device__ __forceinline__ void wire_clip(double p0, double k, double q0, double q1, double err, double& lo, double& hi) {
   const double l = q0 - err - p0, h = q1 + err - p0;
   if (k == 0.0) {
     if (l > 0.0 || h < 0.0) hi = lo - 1.0;
@@ -314,18 +325,18 @@ __device__ __forceinline__ void wire_clip(double p0, double k, double q0, double
   hi = fmin(hi, fmax(i0, i1));
 }
 
-// Every tile a walked step of the wire can fall in (and a few beside it): along the
-// major axis a tile at a time, the tiles its steps there can reach on the other.
+// Every tile a walked step (first to last) of the wire can fall in (and a few beside
+// it): along the major axis a tile at a time, the tiles its steps there can reach on
+// the other.  w: ax, ay, kx, ky; tx, ty: tiles of the screen.
 template <class F>
-__device__ __forceinline__ void wire_tiles(const WireJob& j, const WireRec& r, F&& visit) {
-  const bool xm = fabsf(r.a.z) == 1.0f;  // unit steps along x
-  const float bx = j.cam.bias[0], by = j.cam.bias[1];
-  const int siz = __float_as_int(r.c.x), tx = j.tiles_x, ty = j.ntiles / j.tiles_x;
-  const double ex = wire_axis_err(r.a.x, r.a.z, siz, bx), ey = wire_axis_err(r.a.y, r.a.w, siz, by);
-  const double px = (double)r.a.x + (double)bx, py = (double)r.a.y + (double)by;
-  const double pm = xm ? px : py, km = xm ? r.a.z : r.a.w, em = xm ? ex : ey;
-  const double pn = xm ? py : px, kn = xm ? r.a.w : r.a.z, en = xm ? ey : ex;
-  const double lo = __float_as_int(r.c.y), hi = __float_as_int(r.c.z), tile = kWireTile, inv = 1.0 / kWireTile;
+__host__ __device__ __forceinline__ void wire_tiles(float4 w, int siz, int first, int last, float bx, float by, int tx, int ty,
+                                                    F&& visit) {
+  const bool xm = fabsf(w.z) == 1.0f;  // unit steps along x
+  const double ex = wire_axis_err(w.x, w.z, siz, bx), ey = wire_axis_err(w.y, w.w, siz, by);
+  const double px = (double)w.x + (double)bx, py = (double)w.y + (double)by;
+  const double pm = xm ? px : py, km = xm ? w.z : w.w, em = xm ? ex : ey;
+  const double pn = xm ? py : px, kn = xm ? w.w : w.z, en = xm ? ey : ex;
+  const double lo = first, hi = last, tile = kWireTile, inv = 1.0 / kWireTile;
   const int nm = xm ? tx : ty, nn = xm ? ty : tx;
   const double m0 = pm + km * lo, m1 = pm + km * hi;
   const int c0 = (int)fmin(fmax(floor((fmin(m0, m1) - em) * inv), 0.0), (double)nm);
@@ -350,8 +361,9 @@ constexpr uint64_t kWireGroupSteps = 12288;
 // Group blockIdx.x's wires, at most one a lane (pw to each of the sixteen waves): set
 // up, then, where their steps are many, counted per tile and listed per tile (as
 // bin_group does for faces); where they are few, drawn into memory, so that the tile
-// pass finds nothing to do.  Wires with no length or a value that is not finite, which
-// have no tiles to find, are drawn, as are all of a group whose entries do not fit.
+// pass finds nothing to do.  Wires with no length, a value that is not finite or steps
+// whose place is not known well enough (wire_listed) have no tiles to find and are
+// drawn, as are all of a group whose entries do not fit.
 __global__ void __launch_bounds__(kBinBlock) k_wire_bin(const WireJob jv) {
   TINA_KERNARG_JOB(WireJob, j, jv);
   extern __shared__ __align__(16) uint32_t lds[];
@@ -390,9 +402,15 @@ __global__ void __launch_bounds__(kBinBlock) k_wire_bin(const WireJob jv) {
   __syncthreads();
   const float sum = ((fabsf(s.ax) + fabsf(s.ay)) + (fabsf(s.kx) + fabsf(s.ky))) +
                     ((fabsf(s.ws0) + fabsf(s.ws1)) + (fabsf(s.Az) + fabsf(s.Bz)));
-  const bool list = steps > 0 && s.siz > 0 && sum < 1e9f;
-  WireRec r;
+  const bool list = steps > 0 && s.siz > 0 && sum < 1e9f &&
+                    wire_listed(s.ax, s.ay, s.kx, s.ky, s.siz, j.cam.bias[0], j.cam.bias[1]);
+  const int last = (int)((int64_t)s.i0 + (int64_t)steps - 1);
+  auto tiles = [&](auto&& visit) {
+    wire_tiles(make_float4(s.ax, s.ay, s.kx, s.ky), s.siz, s.i0, last, j.cam.bias[0], j.cam.bias[1], j.tiles_x, ntiles / j.tiles_x,
+               visit);
+  };
   if (list) {
+    WireRec r;
     r.a = make_float4(s.ax, s.ay, s.kx, s.ky);
     r.b = make_float4(s.ws0, s.ws1, s.Az, s.Bz);
     // z by steps: n / d with n = ws0 Az (1 - c) + ws1 Bz c, d = ws0 (1 - c) + ws1 c, c = i / siz
@@ -402,9 +420,8 @@ __global__ void __launch_bounds__(kBinBlock) k_wire_bin(const WireJob jv) {
     // of the largest terms); both ends in front of the camera, or no bound
     const float mx = fmaxf(s.ws0, s.ws1), mn = fminf(s.ws0, s.ws1);
     const float e = 32.0f * 5.9604645e-8f * mx * (1.0f + fmaxf(fabsf(s.Az), fabsf(s.Bz))) * (1.0f + mx / mn);
-    r.c = make_float4(__int_as_float(s.siz), __int_as_float(s.i0),
-                      __int_as_float((int)((int64_t)s.i0 + (int64_t)steps - 1)), mn > 0.0f ? e : INFINITY);
-    wire_tiles(j, r, [&](int t) { atomicAdd(&cnt[t], 1u); });
+    r.c = make_float4(__int_as_float(s.siz), __int_as_float(s.i0), __int_as_float(last), mn > 0.0f ? e : INFINITY);
+    tiles([&](int t) { atomicAdd(&cnt[t], 1u); });
     j.recs[f] = r;
   }
   draw(s, list ? 0 : steps);
@@ -424,7 +441,7 @@ __global__ void __launch_bounds__(kBinBlock) k_wire_bin(const WireJob jv) {
   }
   for (int t = tid; t < ntiles; t += kBinBlock) chunk_off[t] = base + cnt[t];
   __syncthreads();
-  if (list) wire_tiles(j, r, [&](int t) { j.entries[base + atomicAdd(&cnt[t], 1u)] = (uint32_t)f; });
+  if (list) tiles([&](int t) { j.entries[base + atomicAdd(&cnt[t], 1u)] = (uint32_t)f; });
 }
 
 constexpr int kWireQueue = 128;

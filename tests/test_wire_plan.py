@@ -1,8 +1,10 @@
 """The host's plan of wire calls by tile, compiled from the kernels' own header (no GPU
-call): a group's wires are at most a lane each whatever the device's unit count."""
+call): a group's wires are at most a lane each whatever the device's unit count, and
+the entries of as many wires as go at a time have a count of 32 bits."""
 import os
 import subprocess
 
+import numpy as np
 import pytest
 
 from conftest import ROOT
@@ -15,6 +17,19 @@ MAIN = r'''
 #include <stdlib.h>
 using namespace tina;
 int main(int argc, char** argv) {
+  if (argc == 4 && argv[3][0] == '/') {  // wires (ax ay kx ky siz first last) from a file: tiles of each, -1: drawn
+    const int tx = (atoi(argv[1]) + kWireTile - 1) / kWireTile, ty = (atoi(argv[2]) + kWireTile - 1) / kWireTile;
+    FILE* f = fopen(argv[3], "rb");
+    float4 w;
+    int i[3];
+    while (fread(&w, 16, 1, f) == 1 && fread(i, 4, 3, f) == 3) {
+      long n = 0;
+      const bool listed = wire_listed(w.x, w.y, w.z, w.w, i[0], 0.5f, 0.5f);
+      if (listed) wire_tiles(w, i[0], i[1], i[2], 0.5f, 0.5f, tx, ty, [&](int t) { n += t >= 0 && t < tx * ty ? 1 : 1 << 30; });
+      printf("%%ld\n", listed ? n : -1);
+    }
+    return 0;
+  }
   for (int i = 1; i + 2 < argc; i += 3) {
     const WireScratch w = wire_scratch(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]));
     printf("%%ld %%d %%d\n", (long)w.bytes, w.bytes ? w.room : 0, kBinBlock);
@@ -47,3 +62,36 @@ def test_a_group_has_a_lane_for_every_wire(plan, ncu):
     for nbytes, room, lanes in rows:
         assert -(-room // ncu) <= lanes
         assert nbytes == 0 or room >= 1024
+
+
+@pytest.mark.parametrize('W,H', SCREENS)
+def test_entries_keep_a_count_of_32_bits(plan, tmp_path, W, H):
+    """Wires that start on the screen or beside it and end up to 2^31 pixels away, along
+    both axes and at slopes near one: a listed wire has at most three entries a tile of
+    its major axis, so that the room's wires together stay below 2^32 of them."""
+    tx, ty = -(-W // 32), -(-H // 32)
+    (nbytes, room, _), = plan(W, H, 256)
+    rng = np.random.default_rng(3)
+    n = 600
+    w = np.zeros(n, dtype=[('p', '<f4', 4), ('i', '<i4', 3)])
+    siz = np.exp(rng.uniform(np.log(1.0), np.log(2.0 ** 31 - 1), n))
+    siz[:60], siz[60:120] = 2.0 ** 31 - 1, 7.9e6
+    start = rng.uniform(-0.1, 1.1, (n, 2)) * (W, H)
+    minor = np.where(rng.random(n) < 0.5, rng.choice([-1.0, 0.0, 1.0], n), rng.uniform(-1, 1, n))
+    major = rng.choice([-1.0, 1.0], n)
+    xm = np.abs(minor) == 1.0
+    xm |= rng.random(n) < 0.5
+    w['p'][:, :2] = start
+    w['p'][:, 2], w['p'][:, 3] = np.where(xm, major, minor), np.where(xm, minor, major)
+    w['i'][:, 0] = siz
+    # the walked steps, with the set-up's margin on the major axis
+    a, res = np.where(xm, start[:, 0], start[:, 1]), np.where(xm, W, H)
+    err = 2 + (np.abs(a) + siz + 1 + res) * 1e-6
+    lo = np.clip(np.where(major > 0, -a - err, a - res - err), 0, siz)
+    hi = np.clip(np.where(major > 0, res - a + err, a + err), 0, siz)
+    w['i'][:, 1], w['i'][:, 2] = np.ceil(lo), np.floor(hi)
+    (tmp_path / 'wires').write_bytes(w.tobytes())
+    tiles = np.array(plan(W, H, tmp_path / 'wires'))[:, 0]
+    assert len(tiles) == n and (tiles >= 0).sum() > n / 3 and (tiles < 0).sum() >= 60
+    assert tiles.max() <= 3 * max(tx, ty)
+    assert nbytes == 0 or room * int(3 * max(tx, ty)) < 2 ** 32
