@@ -16,7 +16,8 @@
  *     message.  No C++ exception crosses this boundary.  Calls only enqueue work on
  *     the given stream (a hipStream_t passed as void*; NULL = default stream).
  *   - A context is not thread-safe.  All device scratch is allocated by
- *     tina_ctx_create / tina_ctx_resize, never inside the per-frame calls.
+ *     tina_ctx_create, tina_ctx_reserve, tina_wires_reserve and the batch calls
+ *     that lay out a plan, never inside the per-frame calls.
  */
 #ifndef TINA_HIP_H
 #define TINA_HIP_H
@@ -200,9 +201,11 @@ int tina_raster_wires(tina_ctx *ctx, const float *d_verts, int n, uint32_t id_ba
                       void *stream);
 /* Makes the scratch with which tina_raster_wires takes calls of n wires by screen
  * tiles (65,536 wires and more, 131,072 on screens of up to 524,288 pixels; fewer need
- * none, and without it, or where the memory is short, they are drawn into the depth|id buffer directly, with the same result).
- * Made once per context, at most 60 MB at 1920 x 1080; nothing is made while stream
- * is capturing.  Call it where the wires are bound, outside the frame. */
+ * none, and without it they are drawn into the depth|id buffer directly, with the
+ * same result).  Made once per context, 46 MB at 1920 x 1080.  It allocates device
+ * memory, so call it beside tina_ctx_create and not in a frame; where the memory is
+ * short or stream is capturing it makes nothing, returns TINA_OK and may be called
+ * again. */
 int tina_wires_reserve(tina_ctx *ctx, int n, void *stream);
 
 /* The colour pass of WireframeRaster (wireframe.py:92-95, Shader.blend_color

@@ -40,7 +40,6 @@ class Engine:
         _abi.check(lib.tina_ctx_create(int(res_x), int(res_y), int(maxfaces), ctypes.byref(handle)))
         self._ctx = handle
         self._cap = int(maxfaces)
-        self._wires = 0  # the largest wire count asked for
         self._lib = lib
         # default camera: identity with z flipped, bias (0.5, 0.5)  (engine.py:20-26)
         self.W2V = np.eye(4, dtype=np.float32)
@@ -111,10 +110,9 @@ class Engine:
             self._cap = int(nfaces)
 
     def reserve_wires(self, n):
-        """Scratch for calls of n wires (the native side decides whether they need any)."""
-        if n > self._wires:
-            _abi.check(self._lib.tina_wires_reserve(self._ctx, int(n), _abi.stream_handle()), self._ctx)
-            self._wires = int(n)
+        """Scratch for calls of up to n wires (the native side decides whether they need
+        any, and keeps what it has made).  Not for a frame: it allocates device memory."""
+        _abi.check(self._lib.tina_wires_reserve(self._ctx, int(n), _abi.stream_handle()), self._ctx)
 
     def clear_depth(self):
         """Engine.clear_depth (engine.py:67-70): every key -> (2**30, no face)."""

@@ -33,6 +33,8 @@ class WireframeRaster:
         self._fb = None
         self._mesh = None
         self._own = None
+        # scratch for the most wires this raster takes: made here, so that no frame makes any
+        engine.reserve_wires(self.maxfaces)
 
     @property
     def nwires(self):
@@ -61,7 +63,6 @@ class WireframeRaster:
         self._fb = fb
         self._mesh = mesh
         self.nfaces = n
-        self.engine.reserve_wires(n)
         self.id_base = self.engine._id_cursor
         self.engine._id_cursor += n
 
@@ -73,7 +74,6 @@ class WireframeRaster:
         if self._mesh is self._own and self._fb is not None:
             self._fb = self._own.face_buffers()
             self.nfaces = int(self._fb['nfaces'])
-            self.engine.reserve_wires(self.nfaces)
             self.engine._id_cursor = max(self.engine._id_cursor, self.id_base + self.nfaces)
         else:
             self.set_object(self._own)
