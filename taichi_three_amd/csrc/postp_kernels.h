@@ -107,13 +107,17 @@ k_bloom_blur(const float* __restrict__ src, float* __restrict__ dst, int hw, int
 // a tap, so a tap costs a lane two LDS reads and 3 R operations instead of 2 R reads.
 // Every output sums its taps in the same order: identical results.
 //   along x  a wave per channel of 64 R pixels of one row, staged as three planes
-//            with a word of padding each R (lanes R apart fall on different banks)
+//            with a word of padding each R (lanes R apart fall on different banks) and
+//            written out through them in memory order
 //   along y  a lane per float of the row (3 hw of them), 64 to a workgroup, a wave
 //            per R rows
 // Bound by VALU issue (three operations a tap and output, 8 us a pass at 1080p with
 // its radius of 67); one output a lane was bound by LDS reads.  1080p, radius 67:
-// 21 -> 14 us along x, 26 -> 14 along y (R = 8 along x 18); the whole bloom 65 -> 47,
-// at radius 150 102 -> 72, at 200 (unstaged along y before) 185 -> 84.
+// 19 -> 12 us along x, 26 -> 14 along y (R = 8 along x 18); the whole bloom 60 -> 42,
+// at radius 150 94 -> 66, at 284 (unstaged along y before) 233 -> 98.  At small radii
+// the pass is its memory traffic: lanes that store their own R outputs along x, 12 bytes
+// apart, took 9 us where 4.2 are enough (radius 1 at 1080p: 32.7 us for 29.3 of one
+// output a lane; 27.8 in memory order).
 constexpr int kBlurX = 4, kBlurXSeg = 64 * kBlurX;                  // R along x, pixels a workgroup
 constexpr int kBlurY = 4, kBlurYWaves = 8, kBlurYRows = kBlurY * kBlurYWaves;  // R along y, rows a workgroup
 constexpr size_t kBlurLds = 150 * 1024;
@@ -183,8 +187,7 @@ k_bloom_blur_x(const float* __restrict__ src, float* __restrict__ dst, int hw, i
     }
   }
   __syncthreads();
-  const int c = t >> 6, x = x0 + (t & 63) * R;
-  if (x >= hw) return;
+  const int c = t >> 6, last = min(hw - 1 - x0, kBlurXSeg - 1);      // last pixel of the segment
   const float* const w = lds + c * plane + ((t & 63) + margin) * P;  // this lane's outputs
   float win[R], acc[R];
 #pragma unroll
@@ -201,10 +204,16 @@ k_bloom_blur_x(const float* __restrict__ src, float* __restrict__ dst, int hw, i
 #pragma unroll
         for (int u = 0; u < R; u++) v[u] = q[u];
       });
-  float* o = dst + ((long)y * hw + x) * 3 + c;
+  __syncthreads();  // every window is read: the outputs go out through the planes, in order
 #pragma unroll
-  for (int r = 0; r < R; r++)
-    if (x + r < hw) o[3 * r] = acc[r];
+  for (int r = 0; r < R; r++) lds[c * plane + (t & 63) * P + r] = acc[r];
+  __syncthreads();
+  float* const o = dst + ((long)y * hw + x0) * 3;
+#pragma unroll
+  for (int u = 0; u < R; u++) {
+    const int k = t + 192 * u, px = k / 3;
+    if (px <= last) o[k] = lds[(k - 3 * px) * plane + px + px / R];
+  }
 }
 
 __global__ void __launch_bounds__(64 * kBlurYWaves)
