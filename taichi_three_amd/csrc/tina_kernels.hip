@@ -542,9 +542,9 @@ int tina_raster_wires(tina_ctx* c, const float* d_verts, int n, uint32_t id_base
     }
     return TINA_OK;
   }
-  const int per = wires_per_wave(n, c->ncu);
-  hipLaunchKernelGGL(k_wires, dim3(grid_for(n, (long)per * (kBlock / 64), 16384)), dim3(kBlock), 0, s, d_verts, n, per,
-                     id_base, flags, make_cam(c), (unsigned long long*)c->keys);
+  const int parts = wire_parts_log(n, c->ncu);
+  hipLaunchKernelGGL(k_wires, dim3(grid_for((((long)n + 63) / 64) << parts, kBlock / 64, 16384)), dim3(kBlock), 0, s, d_verts,
+                     n, parts, id_base, flags, make_cam(c), (unsigned long long*)c->keys);
   TINA_LAUNCH(c, "k_wires");
   return TINA_OK;
 }

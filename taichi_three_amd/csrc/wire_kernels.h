@@ -111,11 +111,13 @@ __device__ __forceinline__ bool wire_step(const Cam& cam, const WSetup& s, long 
 }
 
 // Draws the wires of a wave's lanes (count steps of s each) into memory, the steps
-// laid end to end, one a lane.  The first slot whose end is beyond step g owns it:
-// the slots that ended before the window of 64, and the ends marked in it below the
-// lane.  mark, slot: LDS of the wave's own, 64 words each, mark at -1.
+// laid end to end, one a lane: of their windows of 64 steps, the part-th of 2^parts_log
+// runs.  The first slot whose end is beyond step g owns it: the slots that ended before
+// the window, and the ends marked in it below the lane.  mark, slot: LDS of the wave's
+// own, 64 words each, mark at -1.
 __device__ __forceinline__ void wires_to_memory(const Cam& cam, const WSetup& s, uint64_t count, uint32_t id,
-                                                unsigned long long* __restrict__ keys, int* mark, int* slot) {
+                                                unsigned long long* __restrict__ keys, int* mark, int* slot, int part = 0,
+                                                int parts_log = 0) {
   const int lane = __lane_id();
   const unsigned long long live = __ballot(count > 0);
   uint64_t end = count;
@@ -129,8 +131,10 @@ __device__ __forceinline__ void wires_to_memory(const Cam& cam, const WSetup& s,
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
   };
   if (count > 0) slot[below(live)] = lane;
-  int kbase = 0, tag = 0;
-  for (uint64_t g0 = 0; g0 < total; g0 += 64) {
+  const uint64_t windows = (total + 63) >> 6;
+  const uint64_t begin = (windows * (uint64_t)part >> parts_log) << 6, until = (windows * (uint64_t)(part + 1) >> parts_log) << 6;
+  int kbase = __popcll(__ballot(count > 0 && end <= begin)), tag = 0;
+  for (uint64_t g0 = begin; g0 < until; g0 += 64) {
     // windows are told apart by 31 bits of their number: a mark is read in its own
     tag = (tag + 1) & 0x7fffffff;
     if (count > 0 && end - 1 >= g0 && end - 1 < g0 + 64) mark[(int)(end - 1 - g0)] = tag;
@@ -164,32 +168,40 @@ __device__ __forceinline__ void wires_to_memory(const Cam& cam, const WSetup& s,
   wave_sync_lds();
 }
 
-// Every wire into memory, `per` (at most 64) wires a wave at a time.
+// Every wire into memory, 64 of them to 2^parts_log waves.
 __global__ void __launch_bounds__(kBlock)
-k_wires(const float* __restrict__ verts, int n, int per, uint32_t id_base, uint32_t flags, const Cam cam,
+k_wires(const float* __restrict__ verts, int n, int parts_log, uint32_t id_base, uint32_t flags, const Cam cam,
         unsigned long long* __restrict__ keys) {
   __shared__ int s_mark[kBlock], s_slot[kBlock];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const bool clip = (flags & TINA_CLIP) != 0;
   s_mark[threadIdx.x] = -1;
-  for (long f0 = ((long)blockIdx.x * (kBlock / 64) + wave) * per; f0 < n; f0 += (long)gridDim.x * (kBlock / 64) * per) {
+  for (long w = (long)blockIdx.x * (kBlock / 64) + wave; (w >> parts_log) * 64 < n; w += (long)gridDim.x * (kBlock / 64)) {
     WSetup s;
     s.ax = s.ay = s.kx = s.ky = s.ws0 = s.ws1 = s.Az = s.Bz = 0.0f;
     s.siz = s.i0 = 0;
     uint64_t cnt = 0;
-    const long f = f0 + lane;
-    if (lane < per && f < n && !wire_setup(cam, (gf32*)verts, f, clip, s, cnt)) cnt = 0;
-    wires_to_memory(cam, s, cnt, id_base + (uint32_t)f, keys, s_mark + 64 * wave, s_slot + 64 * wave);
+    const long f = (w >> parts_log) * 64 + lane;
+    if (f < n && !wire_setup(cam, (gf32*)verts, f, clip, s, cnt)) cnt = 0;
+    wires_to_memory(cam, s, cnt, id_base + (uint32_t)f, keys, s_mark + 64 * wave, s_slot + 64 * wave,
+                    (int)(w & ((1 << parts_log) - 1)), parts_log);
   }
 }
 
-// Wires a wave for a call of n: 64 waves a CU (eight of them at a time) before a
-// wave takes a second wire.  Against 16 waves a CU: 32 k long wires 256 us for 268,
-// 200 k of 2 px 50 for 47; 64 wires a wave, as before, left 500 wires of 600 px with
-// eight workgroups (147 us; 39 now).
-inline int wires_per_wave(long n, int ncu) {
-  const long p = (n + 64L * ncu - 1) / (64L * ncu);
-  return (int)(p < 1 ? 1 : p > 64 ? 64 : p);
+// Waves (a power of two, log) that share 64 wires of a call of n: each sets all of them
+// up and walks its part of their steps.  Four at least, more while that makes at most
+// 64 waves a CU (16 beyond eight): 64 wires a lane of one wave leave a small call with
+// a few long-running waves, and one wire a wave (the set-up of 63 lanes idle) made
+// 16 k short wires wait for three rounds of waves.  Frames of 1080p, four waves on 64
+// wires / one to thirteen wires a wave / so:
+//   500 of 600 px 146 / 38 / 33 us, 4 k of 600 157 / 83 / 76, 16 k of 2 px 25 / 30 / 26,
+//   16 k of 600 186 / 174 / 167, 60 k of 2 29 / 31 / 28, 200 k of 2 41 / 39 / 39,
+//   200 k of 600 816 / 836 / 817, 500 k of 2 62 / 63 / 60 (two waves 64).
+inline int wire_parts_log(long n, int ncu) {
+  const long chunks = (n + 63) / 64;
+  int l = 2;
+  while (l < 6 && chunks << (l + 1) <= (l < 3 ? 64L : 16L) * ncu) l++;
+  return l;
 }
 
 // ---- wires by tile ---------------------------------------------------------------
