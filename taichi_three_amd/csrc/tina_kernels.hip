@@ -45,7 +45,10 @@ struct tina_ctx {
   uint32_t* cursor = nullptr;     // the binning groups' entry cursor (zero between calls)
   FaceRec* recs = nullptr;
   int ncu = 0;                    // compute units of the device
-  void* wires = nullptr;          // scratch of wire calls by tile (WireScratch), or none
+  void* wires = nullptr;          // scratch of wire calls by tile, laid out by wire_plan, or none
+  WireScratch wire_plan{};
+  void* old_wires[8] = {};        // smaller ones that it took the place of: the room doubles (wire_scratch)
+  int nold_wires = 0;
   // learned-shading fallback queue (kFbSeg segments of fb_segcap pixel indices),
   // its segment counters, and k_shade_nn's resident grid
   uint32_t* fbq = nullptr;
@@ -402,6 +405,7 @@ int tina_ctx_create(int width, int height, int max_faces, tina_ctx** out) {
 int tina_ctx_destroy(tina_ctx* c) {
   if (!c) return TINA_OK;
   free_scratch(c);
+  for (int i = 0; i < c->nold_wires; i++) (void)hipFree(c->old_wires[i]);
   for (void* p : {(void*)c->keys, (void*)c->ctr, (void*)c->cursor, (void*)c->fbq, (void*)c->fbn, (void*)c->span, c->wires})
     if (p) (void)hipFree(p);
   delete c;
@@ -522,7 +526,7 @@ int tina_raster_wires(tina_ctx* c, const float* d_verts, int n, uint32_t id_base
   int rc = flush_clear(c, s);
   if (rc) return rc;
   if (c->wires && wires_by_tile(n, (long)c->W * c->H)) {
-    const WireScratch w = wire_scratch(c->W, c->H, c->ncu);
+    const WireScratch& w = c->wire_plan;
     WireJob j;
     wire_scratch_at(w, c->wires, j);
     j.keys = c->keys;
@@ -552,14 +556,14 @@ int tina_raster_wires(tina_ctx* c, const float* d_verts, int n, uint32_t id_base
 int tina_wires_reserve(tina_ctx* c, int n, void* stream) {
   if (!c) return fail(nullptr, TINA_ERR_INVALID, "ctx is NULL");
   if (n < 0) return fail(c, TINA_ERR_INVALID, "n must be >= 0");
-  if (c->wires || !wires_by_tile(n, (long)c->W * c->H)) return TINA_OK;
+  if (!wires_by_tile(n, (long)c->W * c->H)) return TINA_OK;
+  const WireScratch w = wire_scratch(c->W, c->H, c->ncu, n);
+  if (w.bytes == 0 || (c->wires && c->wire_plan.room >= w.room) || c->nold_wires == 8) return TINA_OK;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing((hipStream_t)stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();
     return TINA_OK;  // no allocation while a graph is recorded: the wires are drawn
   }
-  const WireScratch w = wire_scratch(c->W, c->H, c->ncu);
-  if (w.bytes == 0) return TINA_OK;
   void* p = nullptr;
   if (hipMalloc(&p, w.bytes) != hipSuccess) {
     (void)hipGetLastError();
@@ -570,7 +574,9 @@ int tina_wires_reserve(tina_ctx* c, int n, void* stream) {
     (void)hipFree(p);
     return TINA_OK;  // the wires are drawn
   }
+  if (c->wires) c->old_wires[c->nold_wires++] = c->wires;  // a captured frame may still use it
   c->wires = p;
+  c->wire_plan = w;
   return TINA_OK;
 }
 

@@ -255,45 +255,48 @@ struct WireJob {
   int tiles_x, ntiles, ngroups, per;  // per: wires a group
 };
 
-// Scratch of wire calls by tile: one allocation, kept by the context once a call's
-// count asks for it.  At most kWireRoom wires go at a time, and no more than a lane's
-// one for each lane of a workgroup on every unit; they have kWireEntries entries each
-// (wires of 600 px have about 22); a table of counts and one of offsets for as many
-// groups as the device has units.  1080p: 46 MB.
+// Scratch of wire calls by tile, made for calls of so many wires at a time (room, a power
+// of two): as many groups as have a lane for each, and kWireEntries entries a wire (wires
+// of 600 px have about 22).  1080p: 46 MB for 262,144 wires.  Wires beyond the room are a
+// launch pair of their own, which short ones pay for: frames of 500 k of 2 px 83 us with
+// a room of 262,144, 70 with one of 524,288 (of 600 px 720, 659; 1 M of 15 px 313, 176).
 constexpr int kWireLds = kLdsBudget - 16 * 1024;  // for k_wire_bin's counts by tile (its static LDS is 9 KB)
-constexpr int kWireRoom = 262144, kWireEntries = 24, kWireWords = 2;
+constexpr int kWireRoom = 1 << 18, kWireMaxRoom = 1 << 20, kWireEntries = 24, kWireWords = 2;
 struct WireScratch {
   int tiles_x, ntiles, room;
   size_t gcnt, chunk_cnt, chunk_off, entries, recs, bytes;  // places in bytes; the cursor's words come first
 };
 
-inline WireScratch wire_scratch(int W, int H, int ncu) {
+// Wires a group of a call of n, n at most the scratch's room: a group for every unit, at
+// least 64 wires, at most a lane's one each.
+inline int wires_per_group(int n, int ncu) { return std::min(std::max((n + ncu - 1) / ncu, 64), kBinBlock); }
+
+inline WireScratch wire_scratch(int W, int H, int ncu, int n) {
   WireScratch w;
   w.tiles_x = (W + kWireTile - 1) / kWireTile;
   const long ntiles = (long)w.tiles_x * ((H + kWireTile - 1) / kWireTile);
   w.bytes = 0;
   if (4 * ntiles > kWireLds) return w;
   w.ntiles = (int)ntiles;
+  long room = kWireRoom;
+  while (room < n && room < kWireMaxRoom) room *= 2;
   // the count of all entries has 32 bits: a listed wire has three a tile column or row
   // of its major axis at most (wire_listed)
-  w.room = (int)std::min({(long)kWireRoom, (long)kBinBlock * ncu, 0xFFFFFFFFL / (4L * (w.tiles_x + ntiles / w.tiles_x + 4))});
+  w.room = (int)std::min(room, 0xFFFFFFFFL / (4L * (w.tiles_x + ntiles / w.tiles_x + 4)));
+  const size_t groups = (size_t)std::max(ncu, (w.room + kBinBlock - 1) / kBinBlock);
   auto place = [&](size_t n) {
     const size_t at = w.bytes;
     w.bytes += (n + 255) & ~(size_t)255;
     return at;
   };
   place(4 * (size_t)kWireWords);
-  w.gcnt = place(4 * (size_t)ncu);
-  w.chunk_cnt = place(4 * (size_t)ncu * w.ntiles);
-  w.chunk_off = place(4 * (size_t)ncu * w.ntiles);
+  w.gcnt = place(4 * groups);
+  w.chunk_cnt = place(4 * groups * w.ntiles);
+  w.chunk_off = place(4 * groups * w.ntiles);
   w.entries = place(4 * (size_t)w.room * kWireEntries);
   w.recs = place(sizeof(WireRec) * (size_t)w.room);
   return w;
 }
-
-// Wires a group for n of them, n at most the scratch's room: a group for every unit,
-// 64 wires at least.  Never more than k_wire_bin has lanes.
-inline int wires_per_group(int n, int ncu) { return std::max((n + ncu - 1) / ncu, 64); }
 
 inline void wire_scratch_at(const WireScratch& w, void* base, WireJob& j) {
   char* const b = (char*)base;

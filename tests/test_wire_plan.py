@@ -30,9 +30,16 @@ int main(int argc, char** argv) {
     }
     return 0;
   }
-  for (int i = 1; i + 2 < argc; i += 3) {
-    const WireScratch w = wire_scratch(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]));
-    printf("%%ld %%d %%d\n", (long)w.bytes, w.bytes ? w.room : 0, kBinBlock);
+  for (int i = 1; i + 3 < argc; i += 4) {
+    const int ncu = atoi(argv[i + 2]);
+    const WireScratch w = wire_scratch(atoi(argv[i]), atoi(argv[i + 1]), ncu, atoi(argv[i + 3]));
+    if (!w.bytes) {
+      printf("0 0 0 0 0\n");
+      continue;
+    }
+    const int per = wires_per_group(w.room, ncu);
+    printf("%%ld %%d %%d %%d %%ld\n", (long)w.bytes, w.room, per - kBinBlock, (w.room + per - 1) / per,
+           (long)((w.chunk_off - w.chunk_cnt) / 4 / w.ntiles));
   }
   return 0;
 }
@@ -55,13 +62,16 @@ def plan(tmp_path_factory):
 
 @pytest.mark.parametrize('ncu', [16, 32, 64, 80, 128, 256, 304])
 def test_a_group_has_a_lane_for_every_wire(plan, ncu):
-    """k_wire_bin holds one wire a lane: on a device of fewer units than 256 a launch
-    takes fewer wires, so that its groups stay as long as the workgroup."""
-    rows = plan(*[x for W, H in SCREENS for x in (W, H, ncu)])
-    assert len(rows) == len(SCREENS) and sum(r[0] > 0 for r in rows) >= 6
-    for nbytes, room, lanes in rows:
-        assert -(-room // ncu) <= lanes
-        assert nbytes == 0 or room >= 1024
+    """k_wire_bin holds one wire a lane: where there are more wires than a lane each on
+    every unit, there are more groups, each as long as the workgroup, and rows for them."""
+    counts = (65536, 200000, 500000, 1 << 20, 3000000)
+    rows = plan(*[x for W, H in SCREENS for n in counts for x in (W, H, ncu, n)])
+    assert len(rows) == len(SCREENS) * len(counts) and sum(r[0] > 0 for r in rows) >= 30
+    for (nbytes, room, over, groups, tables), n, (W, H) in zip(rows, counts * len(SCREENS),
+                                                               [s for s in SCREENS for _ in counts]):
+        assert over <= 0 and groups <= tables
+        # one launch takes the whole call, up to 2^20 wires and what 32 bits of entries allow
+        assert nbytes == 0 or room >= min(n, 1 << 20) or room >= 2 ** 32 // (4 * (-(-W // 32) + -(-H // 32) + 5))
 
 
 @pytest.mark.parametrize('W,H', SCREENS)
@@ -70,7 +80,7 @@ def test_entries_keep_a_count_of_32_bits(plan, tmp_path, W, H):
     both axes and at slopes near one: a listed wire has at most three entries a tile of
     its major axis, so that the room's wires together stay below 2^32 of them."""
     tx, ty = -(-W // 32), -(-H // 32)
-    (nbytes, room, _), = plan(W, H, 256)
+    (nbytes, room, *_), = plan(W, H, 256, 1 << 20)
     rng = np.random.default_rng(3)
     n = 600
     w = np.zeros(n, dtype=[('p', '<f4', 4), ('i', '<i4', 3)])
