@@ -140,7 +140,8 @@ unsigned grid_for(long n, long per_block, unsigned cap) {
 void allow_big_lds() {
   static const bool done = [] {
     (void)hipFuncSetAttribute((const void*)k_bin, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBudget);
-    (void)hipFuncSetAttribute((const void*)k_wire_bin, hipFuncAttributeMaxDynamicSharedMemorySize, kWireLds);
+    (void)hipFuncSetAttribute((const void*)k_wire_bin<false>, hipFuncAttributeMaxDynamicSharedMemorySize, kWireLds);
+    (void)hipFuncSetAttribute((const void*)k_wire_bin<true>, hipFuncAttributeMaxDynamicSharedMemorySize, kWireLds);
     (void)hipFuncSetAttribute((const void*)k_bloom_blur_x, hipFuncAttributeMaxDynamicSharedMemorySize, kBlurLds);
     (void)hipFuncSetAttribute((const void*)k_bloom_blur_y, hipFuncAttributeMaxDynamicSharedMemorySize, kBlurLds);
     (void)hipFuncSetAttribute((const void*)k_bbin, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBudget);
@@ -534,12 +535,11 @@ int tina_raster_wires(tina_ctx* c, const float* d_verts, int n, uint32_t id_base
     j.flags = flags;
     allow_big_lds();
     for (int f0 = 0; f0 < n; f0 += w.room) {
-      j.verts = d_verts + 6 * (size_t)f0;
-      j.n = std::min(n - f0, w.room);
-      j.id_base = id_base + (uint32_t)f0;
-      j.per = wires_per_group(j.n, c->ncu);
-      j.ngroups = (j.n + j.per - 1) / j.per;
-      hipLaunchKernelGGL(k_wire_bin, dim3(j.ngroups), dim3(kBinBlock), (size_t)j.ntiles * 4, s, j);
+      wire_job_range(j, d_verts, id_base, f0, std::min(n - f0, w.room), c->ncu);
+      if (j.ngroups > c->ncu)
+        hipLaunchKernelGGL(k_wire_bin<true>, dim3(j.ngroups), dim3(kBinBlock), (size_t)j.ntiles * 4, s, j);
+      else
+        hipLaunchKernelGGL(k_wire_bin<false>, dim3(j.ngroups), dim3(kBinBlock), (size_t)j.ntiles * 4, s, j);
       TINA_LAUNCH(c, "k_wire_bin");
       launch_wire_tile(j, c->ncu, s);
       TINA_LAUNCH(c, "k_wire_tile");
@@ -569,7 +569,7 @@ int tina_wires_reserve(tina_ctx* c, int n, void* stream) {
     (void)hipGetLastError();
     return TINA_OK;  // the wires are drawn
   }
-  if (hipMemset(p, 0, kWireWords * sizeof(uint32_t)) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
+  if (hipMemset(p, 0, kWireHead) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
     (void)hipGetLastError();
     (void)hipFree(p);
     return TINA_OK;  // the wires are drawn
