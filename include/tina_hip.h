@@ -202,10 +202,11 @@ int tina_raster_wires(tina_ctx *ctx, const float *d_verts, int n, uint32_t id_ba
 /* Makes the scratch with which tina_raster_wires takes calls of n wires by screen
  * tiles (65,536 wires and more, 131,072 on screens of up to 524,288 pixels; fewer need
  * none, and without it they are drawn into the depth|id buffer directly, with the
- * same result).  46 MB at 1920 x 1080 for up to 262,144 wires, twice and four times that
- * for as many more (1,048,576 go at a time); kept by the context, as is a smaller one
- * made before.  It allocates device memory, so call it beside tina_ctx_create and not in
- * a frame; where the memory is short or stream is capturing it makes nothing, returns
+ * same result).  46 MB at 1920 x 1080 and 83 at 3840 x 2160 for up to 262,144 wires,
+ * twice and four times that for as many more (1,048,576 go at a time); kept by the
+ * context, as is a smaller one made before.  It allocates device memory, so call it
+ * beside tina_ctx_create and not in a frame; where the memory is short or stream is
+ * capturing it makes nothing, returns
  * TINA_OK and may be called again. */
 int tina_wires_reserve(tina_ctx *ctx, int n, void *stream);
 

@@ -267,15 +267,17 @@ struct WireJob {
 };
 
 // Scratch of wire calls by tile, made for calls of so many wires at a time (room, a power
-// of two): as many groups as have a lane for each, and kWireEntries entries a wire (wires
-// of 600 px have about 22).  1080p: 46 MB for 262,144 wires.  Wires beyond the room are a
+// of two): as many groups as have a lane for each, and entries for a quarter of the
+// screen's tile columns and rows a wire, 24 to 64 (random wires over the whole screen have
+// about as many: 22 at 1080p, 44 at 3840 x 2160, where 24 left most of 200 k such wires to
+// be drawn, 1,917 us a frame for 628).  1080p: 46 MB for 262,144 wires.  Wires beyond the room are a
 // launch pair of their own, which short ones pay for: frames of 500 k of 2 px 83 us with
 // a room of 262,144, 70 with one of 524,288 (of 600 px 720, 659; 1 M of 15 px 313, 176).
 constexpr int kWireLds = kLdsBudget - 16 * 1024;  // for k_wire_bin's counts by tile (its static LDS is 9 KB)
-constexpr int kWireRoom = 1 << 18, kWireMaxRoom = 1 << 20, kWireEntries = 24;
+constexpr int kWireRoom = 1 << 18, kWireMaxRoom = 1 << 20;
 constexpr size_t kWireHead = 512;  // bytes at the front that start at zero: the cursor and, on another line, `listed`
 struct WireScratch {
-  int tiles_x, ntiles, room;
+  int tiles_x, ntiles, room, entries_a_wire;
   size_t gcnt, chunk_cnt, chunk_off, entries, recs, bytes;  // places in bytes, behind kWireHead
 };
 
@@ -309,7 +311,8 @@ inline WireScratch wire_scratch(int W, int H, int ncu, int n) {
   w.gcnt = place(4 * groups);
   w.chunk_cnt = place(4 * groups * w.ntiles);
   w.chunk_off = place(4 * groups * w.ntiles);
-  w.entries = place(4 * (size_t)w.room * kWireEntries);
+  w.entries_a_wire = std::min(std::max((w.tiles_x + (int)ntiles / w.tiles_x) / 4, 24), 64);
+  w.entries = place(4 * (size_t)w.room * w.entries_a_wire);
   w.recs = place(sizeof(WireRec) * (size_t)w.room);
   return w;
 }
@@ -323,7 +326,7 @@ inline void wire_scratch_at(const WireScratch& w, void* base, WireJob& j) {
   j.chunk_off = (uint32_t*)(b + w.chunk_off);
   j.entries = (uint32_t*)(b + w.entries);
   j.recs = (WireRec*)(b + w.recs);
-  j.cap = (uint32_t)w.room * kWireEntries;
+  j.cap = (uint32_t)w.room * (uint32_t)w.entries_a_wire;
   j.tiles_x = w.tiles_x;
   j.ntiles = w.ntiles;
 }
