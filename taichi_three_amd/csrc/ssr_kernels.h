@@ -220,12 +220,14 @@ __device__ __forceinline__ void material_sample(const tina_material& m, const Sl
   for (int i = nfac - 1; i >= 0; i--) wei = vmul(wei, fac_stack[i]);
 }
 
-// mapply_pos for a march step: as mapply_pos to the bit wherever a component lies
-// in [-1, 1] (and outside it where that is outside or NaN), with the range test
-// on the divisor alone.  A numerator below the shared-divisor division's range
-// gives a quotient below 2^-59 that may differ in its last bit, which neither the
-// pixel nor a depth comparison can see; one above it, or infinite, gives a
-// quotient outside [-1, 1] or a NaN.
+// mapply_pos for a march step, with the range test on the divisor alone: as
+// mapply_pos to the bit wherever a component lies between 2^-50 and 1 in magnitude,
+// outside [-1, 1] or NaN where that is.  The quotient's two corrections are exact as
+// long as their remainders are no subnormals, for numerators down to 2^-110.  A smaller
+// one over a divisor of at least 2^-60 gives a quotient below 2^-50, which may differ in
+// its last bit: added to 0.5 for the pixel, or compared with depths a multiple of 2^-30
+// apart, it is the same.  A numerator above the shared division's range, or infinite,
+// gives a quotient outside [-1, 1] or a NaN.
 __device__ __forceinline__ V3 march_project(const float* __restrict__ M, V3 p) {
   float r0, r1, r2, w;
   mapply1(M, p.x, p.y, p.z, r0, r1, r2, w);
@@ -301,9 +303,12 @@ struct SsrArgs {
 };
 
 // A pixel's draws from its object's material.  The fixed programs (Diffuse,
-// Classic, Blinn, PBR) keep what does not change between draws -- the two tangent
-// frames, the mix chance and factors -- in registers; any other tree walks its
-// program (material_sample, whose stacks live in scratch).
+// Classic, Blinn, PBR) work out once what does not change between draws: the two
+// tangent frames, the mix chance and factors.  A draw picks its frame by address, so
+// under Classic, Blinn and PBR the compiler keeps them in scratch (164 bytes a lane,
+// read back by every sample); picked by component they stay in registers, at a wave a
+// SIMD less: 1,351 us for the effects frame below instead of 1,264.  Any other tree
+// walks its program (material_sample, whose stacks live in scratch).
 template <int PROG>
 struct SsrDraw {
   static constexpr int kDraws = PROG == PROG_DIFFUSE ? 2 : 3;  // numbers a sample takes from the stream
