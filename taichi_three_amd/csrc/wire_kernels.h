@@ -209,10 +209,10 @@ inline int wire_parts_log(long n, int ncu) {
 // every tile, k_wire_tile walks each tile's.  What bounds it then is VALU issue in
 // the tile pass (about 45 instructions a step, 70 % of its time) and the tiles over
 // the middle of the screen, which hold most entries.
-// 200 k random wires of 600 px at 1080p: 800 us in memory, 317 by tile (k_wire_bin
-// 60, k_wire_tile 257; tiles of 16 pixels 355, of 64 400).  Two workgroups a CU take
-// tiles in turn: a workgroup per tile is as fast, but 4.8 us for 2.5 when all groups
-// have drawn their wires.
+// 200 k random wires of 600 px at 1080p: 800 us in memory, 313 by tile (k_wire_bin
+// 58, k_wire_tile 255; tiles of 16 pixels some 40 more, of 64 80).  Two workgroups a CU
+// take tiles in turn: a workgroup per tile is as fast, but costs 2 us more when all
+// groups have drawn their wires.
 constexpr int kWireTileLog = 5, kWireTile = 1 << kWireTileLog;
 
 // Calls of this many wires take the two kernels (of twice as many where the keys fit an
